@@ -102,3 +102,24 @@ def test_direct_empty_inputs():
     torch.cuda.synchronize()
     assert torch.count_nonzero(zero).item() == 0
 
+
+
+@pytest.mark.parametrize("turns", [0.0, 0.125, 0.25, 0.5, 0.75, 1.0 - 2.0 ** -30,
+                                   0.375 + 2.0 ** -28, 3.0 * 2.0 ** 20 + 0.125,
+                                   2.0 ** 33 + 0.25, 1.0 / 3.0])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_phase_at_quarter_turns_and_large_arguments(turns, sign):
+    """cos and sin of 2 pi phi at the edges of the quarter-turn reduction and
+    far from zero. l = 1/4 and u = 4 phi make phi exact, so the only error is
+    the series' rounding: two ulps of 1 (measured on the CPU: 2.0e-16)."""
+    from wsclean_amd.direct import direct_invert
+    dev = torch.device("cuda:0")
+    phi = sign * turns
+    uvw = torch.tensor([[4.0 * phi, 0.0, 0.0]], dtype=torch.float64, device=dev)
+    wl = torch.ones(1, dtype=torch.float64, device=dev)
+    frac = phi - round(phi)
+    for v, want in ((1.0, np.cos(2 * np.pi * frac)), (1.0j, np.sin(2 * np.pi * frac))):
+        vis = torch.full((1, 1), v, dtype=torch.complex64, device=dev)
+        img = direct_invert(uvw, wl, vis, 2, 2, 0.25, 0.25).cpu().numpy()
+        # pixel (0, 1): l = (1 - 0) / 4, m = 0
+        assert abs(img[1, 0] - want) <= 4.5e-16

@@ -12,7 +12,7 @@
 // The reference evaluates the same sum per visibility into per-thread layers
 // and remaps once at the end; here one thread owns one pixel (invert) or one
 // visibility (predict) and sums in sample (pixel) order, so results are
-// deterministic. The angle is evaluated with sincospi on 2 phi, whose
+// deterministic. The angle is evaluated in turns (turnSinCos64), whose
 // argument reduction is exact; all arithmetic is FP64.
 #include "hws_internal.h"
 
@@ -79,7 +79,7 @@ directInvertKernel(const double* __restrict__ uvw, const double* __restrict__ wl
     for (int k = 0; k < cnt; ++k) {
       const double phi = sU[k] * l + sV[k] * m + sW[k] * n;
       double s, c;
-      sincospi(2.0 * phi, &s, &c);
+      turnSinCos64(phi, s, c);
       acc += sRe[k] * c + sIm[k] * s;
     }
     __syncthreads();
@@ -183,7 +183,7 @@ directPredictKernel(const double* __restrict__ uvw, const double* __restrict__ w
     for (int k = 0; k < cnt; ++k) {
       const double phi = u * sL[k] + v * sM[k] + w * sN[k];
       double s, c;
-      sincospi(2.0 * phi, &s, &c);
+      turnSinCos64(phi, s, c);
       re += sI[k] * c;
       im += sI[k] * s;
     }

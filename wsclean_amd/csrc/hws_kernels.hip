@@ -784,7 +784,7 @@ __device__ __forceinline__ float2 rotationPhasor(const GridArgs& a,
     return make_float2(cf, sf);
   }
   double s, c;
-  sincos(2.0 * kPi * turns, &s, &c);
+  turnSinCos64(turns, s, c);
   return make_float2(float(c), float(s));
 }
 
