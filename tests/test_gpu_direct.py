@@ -110,8 +110,10 @@ def test_direct_empty_inputs():
 @pytest.mark.parametrize("sign", [1.0, -1.0])
 def test_phase_at_quarter_turns_and_large_arguments(turns, sign):
     """cos and sin of 2 pi phi at the edges of the quarter-turn reduction and
-    far from zero. l = 1/4 and u = 4 phi make phi exact, so the only error is
-    the series' rounding: two ulps of 1 (measured on the CPU: 2.0e-16)."""
+    far from zero. l = 1/4 and u = 4 phi make phi exact, so the errors are the
+    series' rounding (2.0e-16, measured on the CPU) and that of the argument
+    2 pi phi of the expected value (half an ulp of up to pi, 2.2e-16, and as
+    much from pi itself)."""
     from wsclean_amd.direct import direct_invert
     dev = torch.device("cuda:0")
     phi = sign * turns
@@ -122,4 +124,4 @@ def test_phase_at_quarter_turns_and_large_arguments(turns, sign):
         vis = torch.full((1, 1), v, dtype=torch.complex64, device=dev)
         img = direct_invert(uvw, wl, vis, 2, 2, 0.25, 0.25).cpu().numpy()
         # pixel (0, 1): l = (1 - 0) / 4, m = 0
-        assert abs(img[1, 0] - want) <= 4.5e-16
+        assert abs(img[1, 0] - want) <= 7e-16
