@@ -3,9 +3,20 @@
 // the forward rows pass computed from the model image for every layer.
 #include "hws_fft_device.h"
 
+#include <algorithm>
+
 namespace hws {
 
 namespace {
+
+// Two waves per SIMD (256 registers a lane). Left to itself the compiler
+// takes up to 512 at the sizes whose workgroups allow it (below 4096) to hold
+// the layer-independent twiddles, and the one wave left per SIMD waits out
+// every LDS access and barrier: at 2048^2 with 32 layers the fused columns of
+// two real images took 1108 us and take 682, the model rows 547 and 486 us an
+// image (reference precision: 1410 -> 818 and 690 -> 550). Three waves (168
+// registers) spill the sums.
+#define HWS_TWO_WAVES __attribute__((amdgpu_waves_per_eu(2, 2)))
 
 // Backward columns pass (after fftRowsBlockedSparseKernel) fused with
 // projectOnImageAndCorrect (gridding/wstackinggridder.cpp:874-907) for every
@@ -21,7 +32,7 @@ namespace {
 // grid (W / 2, images of the kind); dynamic LDS: the transform buffer and
 // the row bits of the pass's layers.
 template <int N, bool REF, bool CPLX>
-__global__ void __launch_bounds__(kProjectColumns * N / 16)
+__global__ void __launch_bounds__(kProjectColumns * N / 16) HWS_TWO_WAVES
 fftColsProjectKernel(ColsProjectArgs a, const float2* __restrict__ layers,
                      const float2* __restrict__ tw, float* __restrict__ sum,
                      float* __restrict__ comp, float* __restrict__ isum,
@@ -160,23 +171,41 @@ fftColsProjectKernel(ColsProjectArgs a, const float2* __restrict__ layers,
   }
 }
 
+// Rows per workgroup of the model rows pass: the four of a row block, so that
+// every store fills its 32-byte group and the lanes of a wave whole lines.
+// With two rows, whose partner rows another workgroup stored some time later,
+// most of the output reached memory in half groups (4096^2 x 64 layers x four
+// images: 14.3 ms against 11.6; 1024^2 x 32 layers: 156 us against 84).
+constexpr int kModelRows = 4;
+
+// Whether the model rows pass keeps to 128 registers and four waves per SIMD
+// by forming the thread index and the twiddle address anew for each layer;
+// else two waves hold what the compiler hoists out of the layer loop. 1024
+// threads (4096) leave no choice; below, measured: real mixed images 320 us
+// against 359 (2048^2 x 32 layers) and 84 against 93 (1024^2), but complex ones
+// 427 against 373, the reference precision 515 against 496 (both spill), and
+// 512^2 x 16 layers, which does not fill the chip, 24 against 18.
+template <int N, bool REF, bool CPLX>
+constexpr bool kModelLean = N > 2048 || (N >= 1024 && !REF && !CPLX);
+
 // Forward rows pass computed from the model for every layer of the batch
 // (copyImageToLayerAndInverseCorrect, gridding/wstackinggridder.cpp:934-969,
-// then the row transforms): a workgroup owns two rows of one image, reads
+// then the row transforms): a workgroup owns four rows of one image, reads
 // their model values and computes their n' once, and then, layer after
 // layer, forms each cell's w-phased input (modelTerm, as modelCell forms it),
-// transforms the two rows and writes the tile columns the columns pass reads
+// transforms the rows and writes the tile columns the columns pass reads
 // (colNeed: one bit per (layer, tile column); the columns pass skips the
 // others). The cells' model values and n' stay in registers across the
 // layers, so a layer costs the phase, the transform and the stores.
-// grid (H / 2): row pair rp = rows 2 rp, 2 rp + 1, pairs of a four-row block
-// run on one XCD one after the other (their stores fill the same lines).
+// grid (H / 4, layer groups): group blockIdx.y takes perGroup consecutive
+// layers; each XCD takes a contiguous range of row blocks.
 template <int N, bool REF, bool CPLX>
-__global__ void __launch_bounds__(kProjectColumns * N / 16)
-fftRowsModelLayersKernel(float2* __restrict__ data, int H, int nbatch,
+__global__ void __launch_bounds__(kModelRows * N / 16)
+    __attribute__((amdgpu_waves_per_eu(kModelLean<N, REF, CPLX> ? 4 : 2)))
+fftRowsModelLayersKernel(float2* __restrict__ data, int H, int nbatch, int perGroup,
                          const float2* __restrict__ tw, ModelSource ms,
                          const uint32_t* __restrict__ colNeed, int tshift) {
-  constexpr int NF = kProjectColumns;
+  constexpr int NF = kModelRows;
   constexpr int T = NF * N / 16;
   constexpr int B0 = N / 16;
   constexpr int RL = LastStage<N>::R, NSL = LastStage<N>::NS, PERL = 16 / RL;
@@ -215,19 +244,23 @@ fftRowsModelLayersKernel(float2* __restrict__ data, int H, int nbatch,
   // rowBase + layer offset + x * 4 + f
   const size_t rowBase = size_t(y0 >> 2) * 4 * W + size_t(y0 & 3);
   float2 in[16], out[16];
+  const int bEnd = min(nbatch, (int(blockIdx.y) + 1) * perGroup);
 #pragma unroll 1
-  for (int b = 0; b < nbatch; ++b) {
+  for (int b = int(blockIdx.y) * perGroup; b < bEnd; ++b) {
     const int layer = ms.layer0 + b;
     const double w = layerToW(ms.map, layer);
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       in[r] = modelTerm<REF>(re[r], CPLX ? imv[r] : 0.0f, CPLX, w, np[r]);
-    regFft<-1, N, NF>(lds, tw, tid, in, out, [] {});
+    int tl = tid;
+    const float2* twl = tw;
+    if constexpr (kModelLean<N, REF, CPLX>) asm volatile("" : "+v"(tl), "+s"(twl));
+    regFft<-1, N, NF>(lds, twl, tl, in, out, [] {});
     float2* g = data + size_t(b) * HW + rowBase;
     const size_t cbit = size_t(layer) * tilesX;
 #pragma unroll
     for (int q = 0; q < PERL; ++q) {
-      const int bt = tid + q * T;
+      const int bt = tl + q * T;
       const int f = bt % NF, bb = bt / NF;
       const int base = (bb / NSL) * NSL * RL + bb % NSL;
 #pragma unroll
@@ -289,32 +322,45 @@ bool launchColsProjectPow2(hws_gridder* g, const ColsProjectArgs& a, bool cplx,
   return ok;
 }
 
-// Every layer per workgroup, the model and n' read and computed once.
+// Waves that the model rows pass is spread over: two rounds of the two waves a
+// SIMD holds.
+constexpr size_t kModelWaves = 4096;
+
+// Every layer of a group per workgroup, the model and n' read and computed
+// once.
 bool launchModelLayersPow2(hws_gridder* g, float2* data, int nbatch, const float2* tw,
                            const ModelSource& model, const FftSparse& sparse) {
   const int W = g->W, H = g->H;
   const bool ref = model.precision == HWS_PRECISION_REFERENCE;
   const bool cplx = model.cplx != 0;
-  const dim3 mgrid(H / kProjectColumns);
+  // Small images do not fill the chip with one workgroup per row pair
+  // (1024^2: one wave per SIMD), so the layers are dealt to as many groups of
+  // workgroups as bring kModelWaves waves, in groups of at least two layers (a
+  // group computes its rows' n' anew, about the time of one layer).
+  const size_t waves = size_t(H / kModelRows) * size_t((kModelRows * W / 16 + 63) / 64);
+  const int groups = int(std::min<size_t>(size_t(nbatch + 1) / 2,
+                                          std::max<size_t>(1, kModelWaves / waves)));
+  const int per = (nbatch + groups - 1) / groups;
+  const dim3 mgrid(H / kModelRows, (nbatch + per - 1) / per);
   bool ok = false;
   switch (W) {
 #define HWS_MODEL_LAYERS(NN)                                                                   \
   case NN:                                                                                     \
     if (ref && cplx)                                                                           \
       hipLaunchKernelGGL((fftRowsModelLayersKernel<NN, true, true>), mgrid,                    \
-                         dim3(kProjectColumns * NN / 16), 0, g->stream, data, H, nbatch,        \
+                         dim3(kModelRows * NN / 16), 0, g->stream, data, H, nbatch, per,   \
                          tw, model, sparse.colNeed, sparse.tshift);                       \
     else if (ref)                                                                              \
       hipLaunchKernelGGL((fftRowsModelLayersKernel<NN, true, false>), mgrid,                   \
-                         dim3(kProjectColumns * NN / 16), 0, g->stream, data, H, nbatch,        \
+                         dim3(kModelRows * NN / 16), 0, g->stream, data, H, nbatch, per,   \
                          tw, model, sparse.colNeed, sparse.tshift);                       \
     else if (cplx)                                                                             \
       hipLaunchKernelGGL((fftRowsModelLayersKernel<NN, false, true>), mgrid,                   \
-                         dim3(kProjectColumns * NN / 16), 0, g->stream, data, H, nbatch,        \
+                         dim3(kModelRows * NN / 16), 0, g->stream, data, H, nbatch, per,   \
                          tw, model, sparse.colNeed, sparse.tshift);                       \
     else                                                                                       \
       hipLaunchKernelGGL((fftRowsModelLayersKernel<NN, false, false>), mgrid,                  \
-                         dim3(kProjectColumns * NN / 16), 0, g->stream, data, H, nbatch,        \
+                         dim3(kModelRows * NN / 16), 0, g->stream, data, H, nbatch, per,   \
                          tw, model, sparse.colNeed, sparse.tshift);                       \
     ok = true;                                                                                 \
     break;
