@@ -494,7 +494,7 @@ void hws_destroy(hws_gridder* g) {
     freeDev(kp.binStart);
     freeDev(kp.extraStart);
     freeDev(kp.itemStart);
-    freeDev(kp.itemBin);
+    freeDev(kp.items);
     freeDev(kp.occ);
     freeDev(kp.need);
     freeDev(kp.rowLive);

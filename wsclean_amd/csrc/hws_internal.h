@@ -277,8 +277,8 @@ struct KindPlan {
   uint32_t* itemStart = nullptr;   // exclusive scan of all items per bin [nbins + 1]
   uint64_t nWorkItems = 0;
   size_t itemCapacity = 0;
-  uint32_t* itemBin = nullptr;  // bin of every work item [nWorkItems]
-  size_t itemBinCapacity = 0;
+  uint4* items = nullptr;  // {bin, index in the bin, first record, records} [nWorkItems]
+  size_t workItemCapacity = 0;
   uint32_t* occ = nullptr;  // bit per bin: the bin holds records [(nbins + 31) / 32]
   size_t occCapacity = 0;
   // bit per bin: a degridding subgrid reads the tile (the bin or its left,
@@ -326,7 +326,7 @@ struct Plan {
   // column) pairs holding a needed tile, [18 + kind] samples listed as not
   // gridded
   unsigned long long* counters = nullptr;
-  uint32_t* queue = nullptr;  // work-queue head of the running grid launch
+  uint32_t* queue = nullptr;  // work-queue counters of the running grid launch
   // rotating contexts: the gridding phase-centre phasor of every sample
   float2* rot = nullptr;
   size_t rotCapacity = 0;

@@ -524,14 +524,22 @@ binItemsKernel(const uint32_t* __restrict__ binStart, const uint32_t* __restrict
     items[b] = (binStart[b + 1] > binStart[b] ? 1u : 0u) + (extraStart[b + 1] - extraStart[b]);
 }
 
-// Item -> bin table: the bin of every work item (thread per bin; a split
-// bin writes one entry per item).
+// The work items: {bin, item index within the bin, first record, records} of
+// every item (thread per bin; a split bin writes one entry per item), so that
+// the grid and degrid kernels find an item's records with one load instead of
+// a chain of three.
 __global__ void __launch_bounds__(kThreads)
-itemBinsKernel(const uint32_t* __restrict__ itemStart, size_t nbins,
-               uint32_t* __restrict__ itemBin) {
+workItemsKernel(const uint32_t* __restrict__ itemStart, const uint32_t* __restrict__ binStart,
+                size_t nbins, uint32_t chunk, uint4* __restrict__ items) {
   const size_t b = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (b >= nbins) return;
-  for (uint32_t j = itemStart[b], e = itemStart[b + 1]; j < e; ++j) itemBin[j] = uint32_t(b);
+  const uint32_t i0 = itemStart[b], i1 = itemStart[b + 1];
+  if (i0 == i1) return;
+  const uint32_t s0 = binStart[b], s1 = binStart[b + 1];
+  for (uint32_t i = i0; i < i1; ++i) {
+    const uint32_t j = i - i0, start = s0 + j * chunk;
+    items[i] = make_uint4(uint32_t(b), j, start, min(s1 - start, chunk));
+  }
 }
 
 // Occupancy bits: bit b of the array is set when bin b holds records
@@ -633,8 +641,7 @@ needKernel(const uint32_t* __restrict__ occ, size_t nbins, int tilesX, int tiles
 
 // One work item of a pass: bin, item index within the bin (0 = the item
 // that writes the tile) and its record range. The items of the pass's bins
-// [binLo, binHi) are numbered in bin order from itemStart[binLo]; the bin of
-// an item is found by binary search of the offsets.
+// [binLo, binHi) are numbered in bin order from itemStart[binLo].
 struct WorkItem {
   uint32_t bin, j, start, count;
 };
@@ -654,19 +661,9 @@ __device__ __forceinline__ uint32_t ownerOf(const uint32_t* __restrict__ offs, u
   return lo;
 }
 
-__device__ __forceinline__ WorkItem decodeItem(uint32_t item, uint32_t binLo, uint32_t binHi,
-                                               const uint32_t* __restrict__ binStart,
-                                               const uint32_t* __restrict__ itemStart,
-                                               uint32_t chunk,
-                                               const uint32_t* __restrict__ itemBin = nullptr) {
-  WorkItem w;
-  const uint32_t g = itemStart[binLo] + item;
-  w.bin = itemBin ? itemBin[g] : ownerOf(itemStart, binLo, binHi, g);
-  w.j = g - itemStart[w.bin];
-  const uint32_t s0 = binStart[w.bin], s1 = binStart[w.bin + 1];
-  w.start = s0 + w.j * chunk;
-  w.count = min(s1 - w.start, chunk);
-  return w;
+__device__ __forceinline__ WorkItem workItem(const uint4* __restrict__ items, uint32_t i) {
+  const uint4 d = items[i];
+  return WorkItem{d.x, d.y, d.z, d.w};
 }
 
 __device__ __forceinline__ uint32_t passItems(uint32_t binLo, uint32_t binHi,
@@ -858,7 +855,7 @@ template <int NIMG, int TG, bool ACCUM>
 __global__ void __launch_bounds__(kGridThreads)
 gridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
                 const uint32_t* __restrict__ extraStart, const uint32_t* __restrict__ itemStart,
-                const uint32_t* __restrict__ itemBin, const uint2* __restrict__ recs,
+                const uint4* __restrict__ items, const uint2* __restrict__ recs,
                 const float2* __restrict__ vis, const float* __restrict__ ktab,
                 const __half2* __restrict__ khalf, const double* __restrict__ uvw,
                 const double* __restrict__ wl, float2* __restrict__ layers,
@@ -893,7 +890,7 @@ gridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   __syncthreads();
   for (uint32_t item = blockIdx.x; item < nItems; item += gridDim.x) {
     // every lane decodes the item (uniform loads)
-    const WorkItem wi = decodeItem(item, binLo, binHi, binStart, itemStart, a.chunk, itemBin);
+    const WorkItem wi = workItem(items, itemStart[binLo] + item);
     const uint32_t bin = wi.bin, start = wi.start, count = wi.count;
     if (ACCUM && count == 0) continue;  // block-uniform; nothing to add
     const int layer = int(bin / uint32_t(a.tilesPerLayer));
@@ -1059,6 +1056,38 @@ gridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   }
 }
 
+// The work queues of a grid launch: kQueues counters on cache lines of their
+// own (cleared before the launch), each dealing out every n-th work item (n =
+// the queues in use) to the workgroups b, b + n, ... A wave takes its queue's
+// next item when it finishes one, so a few heavy items do not leave most waves
+// idle at the end. One counter for all waves was the bound of the grid
+// kernels: atomics on one address return about every 13 ns, 5 ms for the 390 k
+// items of an image kind at 4096^2 x 64 layers. Measured with one counter and
+// with these (batches loaded ahead, see BatchStream, in both): 7.68 and 7.24 ms
+// there (8.84 before either), 6.26 and 2.63 ms at 6144^2 x 96 layers with 55 M
+// samples, 364 and 103 us at 1024^2 x 32 layers with 3.2 M.
+constexpr uint32_t kQueues = 64, kQueueStride = 32;
+
+struct WorkQueue {
+  uint32_t* head;
+  uint32_t n, i;
+};
+
+__device__ __forceinline__ WorkQueue workQueue(uint32_t* queues) {
+  const uint32_t n = min(kQueues, gridDim.x), i = blockIdx.x % n;
+  return WorkQueue{queues + i * kQueueStride, n, i};
+}
+
+// Requests the wave's next item; ticketItem reads it when it is needed.
+__device__ __forceinline__ uint32_t takeTicket(const WorkQueue& q) {
+  uint32_t v = 0;
+  if ((threadIdx.x & 63u) == 0u) v = atomicAdd(q.head, 1u);
+  return v;
+}
+__device__ __forceinline__ uint32_t ticketItem(const WorkQueue& q, uint32_t ticket) {
+  return uint32_t(__builtin_amdgcn_readfirstlane(int(ticket))) * q.n + q.i;
+}
+
 constexpr int kCellWaves = 4;
 constexpr int kCellThreads = 64 * kCellWaves;
 
@@ -1097,7 +1126,7 @@ template <int NIMG, int T, bool ACCUM, bool PAD, bool ROT>
 __global__ void __launch_bounds__(kCellThreads)
 gridCellsKernel(GridArgs a, const uint32_t* __restrict__ binStart,
                 const uint32_t* __restrict__ extraStart, const uint32_t* __restrict__ itemStart,
-                const uint32_t* __restrict__ itemBin, const uint2* __restrict__ recs,
+                const uint4* __restrict__ items, const uint2* __restrict__ recs,
                 const float2* __restrict__ vis, const float* __restrict__ ktab,
                 const __half2* __restrict__ khalf, const double* __restrict__ uvw,
                 const double* __restrict__ wl, float2* __restrict__ layers,
@@ -1135,20 +1164,14 @@ gridCellsKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
   const uint32_t nItems = passItems(binLo, binHi, itemStart);
   const size_t HW = size_t(a.ga.W) * a.ga.H;
-  // items come from a work queue (a counter the host clears before the
-  // launch): a wave takes the next item when it finishes one, so a few
-  // heavy items do not leave most waves idle at the end. The next index is
-  // requested while the current item runs.
+  // the next item is requested while the current one runs
   (void)wave;
-  auto take = [&]() -> uint32_t {
-    uint32_t v = 0;
-    if (lane == 0) v = atomicAdd(queue, 1u);
-    return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
-  };
+  const WorkQueue wq = workQueue(queue);
+  auto take = [&]() { return ticketItem(wq, takeTicket(wq)); };
   uint32_t next = take();
   while (next < nItems) {
     const uint32_t item = next;
-    const WorkItem wi = decodeItem(item, binLo, binHi, binStart, itemStart, a.chunk, itemBin);
+    const WorkItem wi = workItem(items, itemStart[binLo] + item);
     next = take();
     const uint32_t bin = wi.bin, start = wi.start, count = wi.count;
     if (ACCUM && count == 0) continue;
@@ -1295,6 +1318,138 @@ gridCellsKernel(GridArgs a, const uint32_t* __restrict__ binStart,
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// kk / OS of a record's kernel offset index kk = ky OS + kx < 2^20 with OS <=
+// 1023, by multiply-high: exact while kk OS < 2^32. (OS = 1: ky = kk = 0.)
+__device__ __forceinline__ uint32_t kernelRowDivisor(int OS) {
+  return OS > 1 ? 0xFFFFFFFFu / uint32_t(OS) + 1u : 0u;
+}
+__device__ __forceinline__ int kernelRow(int kk, uint32_t byOS) {
+  return int(__umulhi(uint32_t(kk), byOS));
+}
+
+// What the matrix-core grid kernels gather for one batch of 64 records (one
+// per lane): the visibilities of the kind's images, their weights and the
+// phase-centre phasor. Loaded one batch ahead (loadBatch), used when the batch
+// is staged (batchValue).
+template <int NIMG>
+struct BatchValues {
+  float2 v[NIMG];
+  float w[NIMG];
+  float2 ph;
+};
+
+template <int NIMG, bool ROT>
+__device__ __forceinline__ BatchValues<NIMG> loadBatch(const GridArgs& a,
+                                                       const float2* __restrict__ vis, uint2 rec,
+                                                       bool valid) {
+  BatchValues<NIMG> b;
+  b.ph = make_float2(1.0f, 0.0f);
+#pragma unroll
+  for (int gi = 0; gi < NIMG; ++gi) {
+    b.v[gi] = make_float2(0.0f, 0.0f);
+    b.w[gi] = 1.0f;
+  }
+  if (valid) {
+    const uint32_t idx = rec.x & 0x3FFFFFFFu;
+#pragma unroll
+    for (int gi = 0; gi < NIMG; ++gi)
+      b.v[gi] = vis[size_t(idx) * a.nImgTotal + a.imgs.idx[gi]];
+    if (a.cw) {
+#pragma unroll
+      for (int gi = 0; gi < NIMG; ++gi) b.w[gi] = a.cw[size_t(idx) * a.nImgTotal + a.imgs.idx[gi]];
+    }
+    if (ROT) b.ph = a.rot[idx];
+  }
+  return b;
+}
+
+// The visibility of image slot gi as it is gridded: weighted, rotated to the
+// phase centre, conjugated where its sample was folded.
+template <int NIMG, bool ROT>
+__device__ __forceinline__ float2 batchValue(const GridArgs& a, const BatchValues<NIMG>& b,
+                                             uint2 rec, int gi) {
+  float2 x = b.v[gi];
+  if (a.cw) x = make_float2(x.x * b.w[gi], x.y * b.w[gi]);
+  if (ROT) x = rotateBy(x, b.ph);
+  if (rec.x >> 31) x.y = -x.y;
+  return x;
+}
+
+// The batches of a wave's work items in turn, loaded ahead: while a batch is
+// staged and multiplied, the records of the next one (of the same item or of
+// the next) and then its visibilities are on their way, and the item after
+// that is taken from the queue. Most items hold a few dozen records, so
+// without this a wave waits out four dependent memory latencies per item.
+template <int NIMG, bool ROT>
+struct BatchStream {
+  WorkItem item, next;      // this item and the one after (count 0: none)
+  uint32_t nextIndex, ticket, b0;
+  uint2 rec, recNext;
+  bool validNext, last;
+  BatchValues<NIMG> val, valNext;
+};
+
+// Takes the wave's first items and loads their first batch; false if there is
+// none.
+template <int NIMG, bool ROT>
+__device__ __forceinline__ bool firstBatch(BatchStream<NIMG, ROT>& s, const GridArgs& a,
+                                           const uint4* __restrict__ items, uint32_t base,
+                                           uint32_t nItems, const uint2* __restrict__ recs,
+                                           const float2* __restrict__ vis,
+                                           const WorkQueue& queue) {
+  const uint32_t i = ticketItem(queue, takeTicket(queue));
+  if (i >= nItems) return false;
+  s.item = workItem(items, base + i);
+  s.ticket = takeTicket(queue);
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool valid = lane < s.item.count;
+  s.rec = make_uint2(0u, 0u);
+  if (valid) s.rec = recs[s.item.start + lane];
+  s.nextIndex = ticketItem(queue, s.ticket);
+  s.next = WorkItem{0u, 0u, 0u, 0u};
+  if (s.nextIndex < nItems) s.next = workItem(items, base + s.nextIndex);
+  s.ticket = takeTicket(queue);
+  s.b0 = 0u;
+  s.val = loadBatch<NIMG, ROT>(a, vis, s.rec, valid);
+  return true;
+}
+
+// Starts loading the records of the batch after this one.
+template <int NIMG, bool ROT>
+__device__ __forceinline__ void loadNextRecords(BatchStream<NIMG, ROT>& s,
+                                                const uint2* __restrict__ recs) {
+  s.last = s.b0 + 64u >= s.item.count;
+  const uint32_t start = s.last ? s.next.start : s.item.start + s.b0 + 64u;
+  const uint32_t count = s.last ? s.next.count : s.item.count - s.b0 - 64u;
+  const uint32_t lane = threadIdx.x & 63u;
+  s.validNext = lane < count;
+  s.recNext = make_uint2(0u, 0u);
+  if (s.validNext) s.recNext = recs[start + lane];
+}
+
+// Moves to the batch after this one; false when the wave has no more.
+template <int NIMG, bool ROT>
+__device__ __forceinline__ bool advance(BatchStream<NIMG, ROT>& s,
+                                        const uint4* __restrict__ items, uint32_t base,
+                                        uint32_t nItems, const WorkQueue& queue) {
+  if (s.last) {
+    if (s.nextIndex >= nItems) return false;
+    s.item = s.next;
+    s.b0 = 0u;
+    s.nextIndex = ticketItem(queue, s.ticket);
+    s.next = WorkItem{0u, 0u, 0u, 0u};
+    if (s.nextIndex < nItems) {
+      s.next = workItem(items, base + s.nextIndex);
+      s.ticket = takeTicket(queue);
+    }
+  } else {
+    s.b0 += 64u;
+  }
+  s.rec = s.recNext;
+  s.val = s.valNext;
+  return true;
+}
+
 // The tile of a bin as a matrix product: with A[y][r] = v_r * yKernel_r[y -
 // y0_r] and B[r][x] = xKernel_r[x - x0_r] (zero outside record r's
 // footprint), the gridded 16 x 16 tile is G = sum_r A[.][r] B[r][.] = A B,
@@ -1314,7 +1469,7 @@ template <int NIMG, bool ACCUM, bool ROT>
 __global__ void __launch_bounds__(kMfmaThreads)
 gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
                const uint32_t* __restrict__ extraStart, const uint32_t* __restrict__ itemStart,
-               const uint32_t* __restrict__ itemBin, const uint2* __restrict__ recs,
+               const uint4* __restrict__ items, const uint2* __restrict__ recs,
                const float2* __restrict__ vis, const float* __restrict__ ktab,
                const __half2* __restrict__ khalf, const double* __restrict__ uvw,
                const double* __restrict__ wl, float2* __restrict__ layers,
@@ -1350,52 +1505,37 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
   const uint32_t nItems = passItems(binLo, binHi, itemStart);
   const size_t HW = size_t(a.ga.W) * a.ga.H;
-  auto take = [&]() -> uint32_t {
-    uint32_t v = 0;
-    if (lane == 0) v = atomicAdd(queue, 1u);
-    return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
-  };
-  uint32_t next = take();
-  while (next < nItems) {
-    const uint32_t item = next;
-    const WorkItem wi = decodeItem(item, binLo, binHi, binStart, itemStart, a.chunk, itemBin);
-    next = take();
-    const uint32_t bin = wi.bin, start = wi.start, count = wi.count;
-    if (ACCUM && count == 0) continue;
-    floatx4 acc[2 * NIMG];
+  const uint32_t base = itemStart[binLo];
+  const uint32_t byOS = kernelRowDivisor(OS);
+  BatchStream<NIMG, ROT> bs;
+  const WorkQueue wq = workQueue(queue);
+  if (!firstBatch(bs, a, items, base, nItems, recs, vis, wq)) return;
+  floatx4 acc[2 * NIMG];
 #pragma unroll
-    for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t b0 = 0; b0 < count; b0 += 64u) {
+  for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  do {
+    {
+      loadNextRecords(bs, recs);
       // stage 64 records (zero samples past the end: their A rows vanish)
+      const uint2 rec = bs.rec;
       int pos = 0;
       float2 v[NIMG];
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) v[gi] = make_float2(0.0f, 0.0f);
-      const uint32_t it = b0 + uint32_t(lane);
-      if (it < count) {
-        const uint2 rec = recs[start + it];
-        const uint32_t idx = rec.x & 0x3FFFFFFFu;
-        const bool conj = (rec.x >> 31) != 0;
+      if (bs.b0 + uint32_t(lane) < bs.item.count) {
         const int kk = int(rec.y >> 12);
-        const int ky = kk / OS, kx = kk - ky * OS;
+        const int ky = kernelRow(kk, byOS), kx = kk - ky * OS;
         const int xs = int(rec.y & 63u), ys = int((rec.y >> 6) & 63u);
         pos = (kx * rowLen + (T - 1) + (K - 1) - xs) |
               ((ky * rowLen + (T - 1) + (K - 1) - ys) << 16);
-        float2 ph = make_float2(1.0f, 0.0f);
-        if (ROT) ph = a.rot[idx];
 #pragma unroll
-        for (int gi = 0; gi < NIMG; ++gi) {
-          float2 x = weighted(a, vis[size_t(idx) * a.nImgTotal + a.imgs.idx[gi]], idx,
-                              a.imgs.idx[gi]);
-          if (ROT) x = rotateBy(x, ph);
-          if (conj) x.y = -x.y;
-          v[gi] = x;
-        }
+        for (int gi = 0; gi < NIMG; ++gi) v[gi] = batchValue<NIMG, ROT>(a, bs.val, rec, gi);
       }
       myPos[lane] = pos;
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) myVis[lane * NIMG + gi] = v[gi];
       waveSync();
+      bs.valNext = loadBatch<NIMG, ROT>(a, vis, bs.recNext, bs.validNext);
       // all 64 staged records, sixteen (four groups of four) per round with
       // their LDS reads issued before the first product; the staging is zero
       // past the item's end, and a fully unrolled batch keeps the
@@ -1432,6 +1572,9 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       }
       waveSync();  // the staging is rewritten next batch
     }
+    if (!bs.last) continue;
+    const WorkItem wi = bs.item;
+    const uint32_t bin = wi.bin;
     // lane owns column li, rows 4 lk .. 4 lk + 3
     if (wi.j > 0) {
       float2* dst = partials + size_t(extraStart[bin] + wi.j - 1u) * size_t(NIMG * T2);
@@ -1477,7 +1620,26 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
         }
       }
     }
-  }
+#pragma unroll
+    for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  } while (advance(bs, items, base, nItems, wq));
+}
+
+// The largest of the wave's non-negative values, on every lane: shifted
+// within the rows of 16 lanes, then across them (DPP, no LDS round trips), and
+// read from the last lane.
+__device__ __forceinline__ float waveMax(float v) {
+  int m = __float_as_int(v);  // (non-negative floats order as integers)
+#define HWS_DPP_MAX(ctrl, rows) \
+  m = max(m, __builtin_amdgcn_update_dpp(0, m, ctrl, rows, 0xf, false))
+  HWS_DPP_MAX(0x111, 0xf);  // row_shr:1
+  HWS_DPP_MAX(0x112, 0xf);  // row_shr:2
+  HWS_DPP_MAX(0x114, 0xf);  // row_shr:4
+  HWS_DPP_MAX(0x118, 0xf);  // row_shr:8
+  HWS_DPP_MAX(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  HWS_DPP_MAX(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef HWS_DPP_MAX
+  return __int_as_float(__builtin_amdgcn_readlane(m, 63));
 }
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -1551,9 +1713,10 @@ __device__ __forceinline__ uint32_t lowParts(float x0, float x1, uint32_t h) {
 // not fit the LDS (above 221 at K = 7); the values are the same.
 template <int NIMG, bool ACCUM, bool ROT, bool GT>
 __global__ void __launch_bounds__(kMfmaThreads)
+    __attribute__((amdgpu_waves_per_eu(NIMG <= 2 ? 4 : 3)))
 gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
                   const uint32_t* __restrict__ extraStart, const uint32_t* __restrict__ itemStart,
-                  const uint32_t* __restrict__ itemBin, const uint2* __restrict__ recs,
+                  const uint4* __restrict__ items, const uint2* __restrict__ recs,
                   const float2* __restrict__ vis, const float* __restrict__ ktab,
                   const float* __restrict__ gkt, const uint32_t* __restrict__ gkp,
                   float2* __restrict__ layers, float2* __restrict__ partials,
@@ -1583,47 +1746,31 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
   const uint32_t nItems = passItems(binLo, binHi, itemStart);
   const size_t HW = size_t(a.ga.W) * a.ga.H;
-  auto take = [&]() -> uint32_t {
-    uint32_t v = 0;
-    if (lane == 0) v = atomicAdd(queue, 1u);
-    return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
-  };
-  uint32_t next = take();
-  while (next < nItems) {
-    const uint32_t item = next;
-    const WorkItem wi = decodeItem(item, binLo, binHi, binStart, itemStart, a.chunk, itemBin);
-    next = take();
-    const uint32_t bin = wi.bin, start = wi.start, count = wi.count;
-    if (ACCUM && count == 0) continue;
-    floatx4 acc[2 * NIMG];
+  const uint32_t base = itemStart[binLo];
+  const uint32_t byOS = kernelRowDivisor(OS);
+  BatchStream<NIMG, ROT> bs;
+  const WorkQueue wq = workQueue(queue);
+  if (!firstBatch(bs, a, items, base, nItems, recs, vis, wq)) return;
+  floatx4 acc[2 * NIMG];
 #pragma unroll
-    for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t b0 = 0; b0 < count; b0 += 64u) {
+  for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  do {
+    {
+      loadNextRecords(bs, recs);
       // stage 64 records (zero samples past the end: their A rows vanish)
+      const uint2 rec = bs.rec;
       int pos = 0;
       float2 v[NIMG];
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) v[gi] = make_float2(0.0f, 0.0f);
-      const uint32_t it = b0 + uint32_t(lane);
-      if (it < count) {
-        const uint2 rec = recs[start + it];
-        const uint32_t idx = rec.x & 0x3FFFFFFFu;
-        const bool conj = (rec.x >> 31) != 0;
+      if (bs.b0 + uint32_t(lane) < bs.item.count) {
         const int kk = int(rec.y >> 12);
-        const int ky = kk / OS, kx = kk - ky * OS;
+        const int ky = kernelRow(kk, byOS), kx = kk - ky * OS;
         const int xs = int(rec.y & 63u), ys = int((rec.y >> 6) & 63u);
         pos = (kx * rowLen + (T - 1) + (K - 1) - xs) |
               ((ky * rowLen + (T - 1) + (K - 1) - ys) << 16);
-        float2 ph = make_float2(1.0f, 0.0f);
-        if (ROT) ph = a.rot[idx];
 #pragma unroll
-        for (int gi = 0; gi < NIMG; ++gi) {
-          float2 x = weighted(a, vis[size_t(idx) * a.nImgTotal + a.imgs.idx[gi]], idx,
-                              a.imgs.idx[gi]);
-          if (ROT) x = rotateBy(x, ph);
-          if (conj) x.y = -x.y;
-          v[gi] = x;
-        }
+        for (int gi = 0; gi < NIMG; ++gi) v[gi] = batchValue<NIMG, ROT>(a, bs.val, rec, gi);
       }
       // each image's scale: 2^e above its largest visibility component in
       // the batch, so that |v yKernel| 2^(kAExp - e - eB) < 2^kAExp (a scale
@@ -1633,8 +1780,7 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) {
         float m = fmaxf(fabsf(v[gi].x), fabsf(v[gi].y));
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        m = waveMax(m);
         int e = 0;
         (void)frexpf(m, &e);  // m < 2^e (0 for m = 0)
         const float down = ldexpf(1.0f, kAExp - e - eB);
@@ -1646,6 +1792,7 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) myVis[lane * NIMG + gi] = v[gi];
       waveSync();
+      bs.valNext = loadBatch<NIMG, ROT>(a, vis, bs.recNext, bs.validNext);
       floatx4 d[2 * NIMG];
 #pragma unroll
       for (int c = 0; c < 2 * NIMG; ++c) d[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1711,6 +1858,9 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
       }
       waveSync();  // the staging is rewritten next batch
     }
+    if (!bs.last) continue;
+    const WorkItem wi = bs.item;
+    const uint32_t bin = wi.bin;
     // lane owns column li, rows 4 lg .. 4 lg + 3
     if (wi.j > 0) {
       float2* dst = partials + size_t(extraStart[bin] + wi.j - 1u) * size_t(NIMG * T2);
@@ -1755,7 +1905,9 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
         }
       }
     }
-  }
+#pragma unroll
+    for (int e = 0; e < 2 * NIMG; ++e) acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  } while (advance(bs, items, base, nItems, wq));
 }
 
 // The visibilities of one primary record from the subgrid around its tile
@@ -1853,9 +2005,9 @@ __device__ __forceinline__ DegridItem degridItem(const GridArgs& a, uint32_t ite
                                                  uint32_t binLo, uint32_t binHi,
                                                  const uint32_t* __restrict__ binStart,
                                                  const uint32_t* __restrict__ itemStart,
-                                                 const uint32_t* __restrict__ itemBin) {
+                                                 const uint4* __restrict__ items) {
   DegridItem d;
-  d.wi = decodeItem(item, binLo, binHi, binStart, itemStart, a.chunk, itemBin);
+  d.wi = workItem(items, itemStart[binLo] + item);
   d.layer = int(d.wi.bin / uint32_t(a.tilesPerLayer));
   const int rem = int(d.wi.bin - uint32_t(d.layer) * uint32_t(a.tilesPerLayer));
   const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
@@ -1926,7 +2078,7 @@ __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkI
 template <int NIMG, int KK>
 __global__ void __launch_bounds__(kThreads)
 degridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
-                  const uint32_t* __restrict__ itemStart, const uint32_t* __restrict__ itemBin,
+                  const uint32_t* __restrict__ itemStart, const uint4* __restrict__ items,
                   const uint2* __restrict__ recs, const float* __restrict__ ktab,
                   const __half2* __restrict__ khalf, const double* __restrict__ uvw,
                   const double* __restrict__ wl, const float2* __restrict__ layers,
@@ -1943,7 +2095,7 @@ degridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   const uint32_t nItems = passItems(binLo, binHi, itemStart);
   for (uint32_t item = blockIdx.x; item < nItems; item += gridDim.x) {
     // every lane decodes the item (uniform loads)
-    const DegridItem d = degridItem(a, item, binLo, binHi, binStart, itemStart, itemBin);
+    const DegridItem d = degridItem(a, item, binLo, binHi, binStart, itemStart, items);
     if (d.wi.count == 0) continue;  // block-uniform
     __syncthreads();  // previous item's readers are done with sub and the queues
     for (int cell = threadIdx.x; cell < sg2; cell += blockDim.x)
@@ -2624,7 +2776,7 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
   if (!pl.counters)
     HWS_TRY(checkHip(g, hipMalloc(&pl.counters, kPlanCounters * sizeof(unsigned long long)),
                      "plan counters"));
-  if (!pl.queue) HWS_TRY(checkHip(g, hipMalloc(&pl.queue, 64 * sizeof(uint32_t)), "plan queue"));
+  if (!pl.queue) HWS_TRY(checkHip(g, hipMalloc(&pl.queue, kQueues * kQueueStride * sizeof(uint32_t)), "plan queue"));
   HWS_TRY(launchFill(g, pl.counters, 0u, 2 * kPlanCounters));
 
   const GeomArgs ga = geomArgs(g);
@@ -2728,8 +2880,8 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
     kp.nItems = total;
     kp.nExtra = totals[1];
     kp.nWorkItems = totals[2];
-    HWS_TRY(ensureAlloc(g, kp.itemBin, kp.itemBinCapacity, size_t(kp.nWorkItems),
-                        "plan item bins"));
+    HWS_TRY(ensureAlloc(g, kp.items, kp.workItemCapacity, size_t(kp.nWorkItems),
+                        "plan work items"));
     const size_t occWords = (pl.nbins + 31) / 32;
     HWS_TRY(ensureAlloc(g, kp.occ, kp.occCapacity, occWords, "plan occupancy"));
     hipLaunchKernelGGL(occupancyKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
@@ -2759,9 +2911,9 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
     hipLaunchKernelGGL(popcountKernel, dim3(blocksFor(colWords)), dim3(kThreads), 0, g->stream,
                        kp.colNeed, colWords, pl.counters + 16 + kind);
     HWS_TRY(checkHip(g, hipGetLastError(), "tile count launch"));
-    hipLaunchKernelGGL(itemBinsKernel, dim3(blocksFor(pl.nbins)), dim3(kThreads), 0, g->stream,
-                       kp.itemStart, pl.nbins, kp.itemBin);
-    HWS_TRY(checkHip(g, hipGetLastError(), "item bin launch"));
+    hipLaunchKernelGGL(workItemsKernel, dim3(blocksFor(pl.nbins)), dim3(kThreads), 0, g->stream,
+                       kp.itemStart, kp.binStart, pl.nbins, pl.chunk, kp.items);
+    HWS_TRY(checkHip(g, hipGetLastError(), "work item launch"));
     HWS_TRY(ensureAlloc(g, kp.recSorted, kp.capacity, size_t(total), "plan sorted records"));
     if (kp.nExtra)
       HWS_TRY(ensureAlloc(g, kp.partials, kp.partialCapacity,
@@ -2897,7 +3049,7 @@ hws_status gridBinned(hws_gridder* g, const float* dVis, int pass, bool accumula
         const unsigned mblocks = unsigned(std::max<uint64_t>(
             1, std::min<uint64_t>((kp.nWorkItems + kMfmaWaves - 1) / kMfmaWaves,
                                   uint64_t(persistentBlocks(g, 8)))));
-        hipLaunchKernelGGL(fillKernel, dim3(1), dim3(64), 0, g->stream, pl.queue, 0u, size_t(1));
+        HWS_TRY(launchFill(g, pl.queue, 0u, kQueues * kQueueStride));
         const bool f16 = mfmaF16(g), gt = f16 && f16TableGlobal(g);
         if (gt && !g->dF16Table)
           return setLastError(g, HWS_ERR_BAD_STATE, "padded kernel table not built");
@@ -2910,16 +3062,16 @@ hws_status gridBinned(hws_gridder* g, const float* dVis, int pass, bool accumula
   if (gt)                                                                                      \
     hipLaunchKernelGGL((gridMfmaF16Kernel<N, ACC, ROT, true>), dim3(mblocks),                   \
                        dim3(kMfmaThreads), lds, g->stream, a, kp.binStart, kp.extraStart,       \
-                       kp.itemStart, kp.itemBin, kp.recSorted, vis, g->dKernel, gkt, gkp,       \
+                       kp.itemStart, kp.items, kp.recSorted, vis, g->dKernel, gkt, gkp,       \
                        layers, kp.partials, pl.queue, g->kernelExp);                            \
   else if (f16)                                                                                \
     hipLaunchKernelGGL((gridMfmaF16Kernel<N, ACC, ROT, false>), dim3(mblocks),                  \
                        dim3(kMfmaThreads), lds, g->stream, a, kp.binStart, kp.extraStart,       \
-                       kp.itemStart, kp.itemBin, kp.recSorted, vis, g->dKernel, nullptr,        \
+                       kp.itemStart, kp.items, kp.recSorted, vis, g->dKernel, nullptr,        \
                        nullptr, layers, kp.partials, pl.queue, g->kernelExp);                   \
   else                                                                                         \
     hipLaunchKernelGGL((gridMfmaKernel<N, ACC, ROT>), dim3(mblocks), dim3(kMfmaThreads), lds,   \
-                       g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.itemBin,      \
+                       g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.items,      \
                        kp.recSorted, vis, g->dKernel, khalf, pl.uvw, pl.wavelengths, layers,    \
                        kp.partials, pl.queue)
 #define HWS_MFMA_CASE(N)                                                                       \
@@ -2953,12 +3105,12 @@ hws_status gridBinned(hws_gridder* g, const float* dVis, int pass, bool accumula
                                   uint64_t(persistentBlocks(g, 8)))));
 #define HWS_CELL_GO(N, TT, ACC, PAD, ROT)                                                   \
   hipLaunchKernelGGL((gridCellsKernel<N, TT, ACC, PAD, ROT>), dim3(cblocks), dim3(kCellThreads), \
-                     lds, g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.itemBin,    \
+                     lds, g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.items,    \
                      kp.recSorted, vis, g->dKernel, khalf, pl.uvw, pl.wavelengths, layers,       \
                      kp.partials, pl.queue)
 #define HWS_CELL_LAUNCH(N, TT, ACC)                \
   do {                                             \
-    hipLaunchKernelGGL(fillKernel, dim3(1), dim3(64), 0, g->stream, pl.queue, 0u, size_t(1)); \
+    HWS_TRY(launchFill(g, pl.queue, 0u, kQueues * kQueueStride)); \
     if (pad && !a.ga.rotate)                       \
       HWS_CELL_GO(N, TT, ACC, true, false);        \
     else if (pad)                                  \
@@ -2994,7 +3146,7 @@ hws_status gridBinned(hws_gridder* g, const float* dVis, int pass, bool accumula
       } else {
 #define HWS_GRID_LAUNCH(N, TG, ACC)                                                           \
   hipLaunchKernelGGL((gridTilesKernel<N, TG, ACC>), dim3(blocks), dim3(kGridThreads), lds,      \
-                     g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.itemBin,        \
+                     g->stream, a, kp.binStart, kp.extraStart, kp.itemStart, kp.items,        \
                      kp.recSorted, vis,                                                         \
                      g->dKernel,                                                                \
                      khalf, pl.uvw, pl.wavelengths, layers, kp.partials)
@@ -3097,7 +3249,7 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
       switch (n) {
 #define HWS_DEGRID_GO(N, KK)                                                                  \
   hipLaunchKernelGGL((degridTilesKernel<N, KK>), dim3(blocks), dim3(kThreads), lds, g->stream,   \
-                     a, kp.binStart, kp.itemStart, kp.itemBin, kp.recSorted, g->dKernel, khalf,  \
+                     a, kp.binStart, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,  \
                      pl.uvw, pl.wavelengths, reinterpret_cast<const float2*>(g->dLayers), out)
 #define HWS_DEGRID_CASE(N)                                                                \
   case N:                                                                                   \
