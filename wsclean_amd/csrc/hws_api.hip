@@ -476,9 +476,9 @@ void hws_destroy(hws_gridder* g) {
   freeFftPlan(g->rowPlan);
   freeFftPlan(g->colPlan);
   Plan& pl = g->plan;
-  freeDev(pl.scanTmp);
   freeDev(pl.scanScratch);
   freeDev(pl.counters);
+  if (pl.hostCounters) (void)hipHostFree(pl.hostCounters);
   freeDev(pl.queue);
   freeDev(pl.rot);
   freeDev(pl.cw);
@@ -495,6 +495,7 @@ void hws_destroy(hws_gridder* g) {
     freeDev(kp.extraStart);
     freeDev(kp.itemStart);
     freeDev(kp.items);
+    freeDev(kp.splitBins);
     freeDev(kp.occ);
     freeDev(kp.need);
     freeDev(kp.rowLive);

@@ -19,7 +19,7 @@
 namespace hws {
 
 constexpr int kMaxImages = 4;
-constexpr int kPlanCounters = 20;
+constexpr int kPlanCounters = 28;
 constexpr int kMaxFftStages = 24;
 constexpr int kMaxKernelSize = 15;
 constexpr int kMaxOversampling = 1023;
@@ -279,6 +279,9 @@ struct KindPlan {
   size_t itemCapacity = 0;
   uint4* items = nullptr;  // {bin, index in the bin, first record, records} [nWorkItems]
   size_t workItemCapacity = 0;
+  uint32_t* splitBins = nullptr;  // bins with extra items, in bin order [nSplit]
+  uint64_t nSplit = 0;
+  size_t splitCapacity = 0;
   uint32_t* occ = nullptr;  // bit per bin: the bin holds records [(nbins + 31) / 32]
   size_t occCapacity = 0;
   // bit per bin: a degridding subgrid reads the tile (the bin or its left,
@@ -315,17 +318,18 @@ struct Plan {
   uint32_t chunk = 0;  // records per work item of the binned kernels
   KindPlan kinds[2];
   // temporaries
-  uint32_t* scanTmp = nullptr;
   uint32_t* scanScratch = nullptr;
-  size_t scanCapacity = 0, scanScratchCapacity = 0;
+  size_t scanScratchCapacity = 0;
   // [kind * 3 + {0: gridded, 1: off grid, 2: off layer}], [6 + kind]: bins used
   // [0..2] gridded / off grid / off layer (real kind), [3..5] the same
   // (complex kind), [6 + kind] bins used, [8 + kind] occupied tiles,
   // [10 + kind] needed tiles, [12 + kind] bins failing the plan check,
   // [14 + kind] live (layer, tile row) pairs, [16 + kind] (layer, tile
   // column) pairs holding a needed tile, [18 + kind] samples listed as not
-  // gridded
+  // gridded, [20 + 4 kind + {0: records, 1: extra items, 2: items, 3: split
+  // bins}]
   unsigned long long* counters = nullptr;
+  unsigned long long* hostCounters = nullptr;  // pinned copy
   uint32_t* queue = nullptr;  // work-queue counters of the running grid launch
   // rotating contexts: the gridding phase-centre phasor of every sample
   float2* rot = nullptr;
@@ -516,7 +520,7 @@ hws_status exclusiveScan(hws_gridder* g, const uint32_t* in, uint32_t* out, size
 hws_status sortRecords(hws_gridder* g, uint32_t*& keys, uint32_t*& keysAlt, uint2*& recs,
                        uint2*& recsAlt, size_t n, int endBit);
 hws_status sortRows(hws_gridder* g, uint32_t*& keys, uint32_t*& keysAlt, uint32_t*& rows,
-                    uint32_t*& rowsAlt, size_t n);
+                    uint32_t*& rowsAlt, size_t n, int endBit);
 hws_status gridPlain(hws_gridder* g, size_t nrow, size_t nchan,
                      const double* dUvw, const double* dWl, const float* dVis,
                      int pass);

@@ -264,19 +264,19 @@ __device__ __forceinline__ bool emission(const GeomArgs& ga, const Placement& p,
 }
 
 // Sort key of a row: the bin of the first tile its middle channel's footprint
-// touches (0xFFFFFFFF when that sample is not gridded). Rows with equal keys
+// touches (noKey, above every bin, when that sample is not gridded). Rows with equal keys
 // have nearly equal uvw, so their samples fall in the same bins channel by
 // channel.
 __global__ void __launch_bounds__(kThreads)
 rowKeyKernel(const double* __restrict__ uvw, const double* __restrict__ wl, size_t nrow,
-             int nchan, GeomArgs ga, LayerMap lm, uint32_t* __restrict__ keys,
+             int nchan, GeomArgs ga, LayerMap lm, uint32_t noKey, uint32_t* __restrict__ keys,
              uint32_t* __restrict__ rows) {
   const size_t r = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (r >= nrow) return;
   const double lambda = wl[nchan / 2];
   const Placement p = place(ga, lm, uvw[r * 3] / lambda, uvw[r * 3 + 1] / lambda,
                             uvw[r * 3 + 2] / lambda);
-  uint32_t key = 0xFFFFFFFFu;
+  uint32_t key = noKey;
   if (p.layer >= 0 && p.onGrid) {
     TileSpan sx, sy;
     footprintSpans(ga, p, sx, sy);
@@ -498,95 +498,234 @@ nanSkippedKernel(const uint32_t* __restrict__ skipped, size_t n, ImgList imgs, i
   for (int gi = 0; gi < imgs.n; ++gi) out[base + imgs.idx[gi]] = make_float2(q, q);
 }
 
-// Work items per bin: a bin of c > 0 records is processed as ceil(c / chunk)
-// items, the first plus (c - 1) / chunk extra ones; an empty bin has none
-// (its tile is cleared before gridding). Pass 1 writes the extra items per bin
-// (and counts the non-empty bins), pass 2 -- after the scan of pass 1 into
-// extraStart -- all items per bin.
-__global__ void __launch_bounds__(kThreads)
-extraItemsKernel(const uint32_t* __restrict__ binStart, size_t nbins, uint32_t chunk,
-                 uint32_t* __restrict__ extra, unsigned long long* __restrict__ nonEmpty) {
-  const size_t b = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  uint32_t c = 0;
-  if (b < nbins) {
-    c = binStart[b + 1] - binStart[b];
-    extra[b] = c > chunk ? (c - 1u) / chunk : 0u;
+// Exclusive prefix of v over the workgroup's kThreads threads (wave scans by
+// shuffles, then the waves' totals through LDS); total = the workgroup's sum.
+// sh holds kThreads / 64 values; a barrier separates it from later use.
+__device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t* sh,
+                                                       uint32_t* total) {
+  constexpr int kWaves = kThreads / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t incl = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
   }
-  const int cnt = __syncthreads_count(b < nbins && c > 0u);
-  if (threadIdx.x == 0 && cnt) atomicAdd(nonEmpty, (unsigned long long)cnt);
+  if (lane == 63) sh[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0u, all = 0u;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t t = sh[w];
+    if (w < wave) before += t;
+    all += t;
+  }
+  *total = all;
+  __syncthreads();
+  return before + incl - v;
 }
 
-__global__ void __launch_bounds__(kThreads)
-binItemsKernel(const uint32_t* __restrict__ binStart, const uint32_t* __restrict__ extraStart,
-               size_t nbins, uint32_t* __restrict__ items) {
-  const size_t b = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b < nbins)
-    items[b] = (binStart[b + 1] > binStart[b] ? 1u : 0u) + (extraStart[b + 1] - extraStart[b]);
+constexpr int kScanItems = 8;
+constexpr int kScanBlock = kThreads * kScanItems;  // values per workgroup of a scan
+
+// The offsets of a plan from its bins' record counts c, in two kernels about
+// one small one: the first record of every bin, its first work item and its
+// first extra item. A bin of c > 0 records is processed as ceil(c / chunk)
+// items, the first plus (c - 1) / chunk extra ones. (Scanning the three arrays
+// one after the other, with the bins' items, bits and cursors set by kernels
+// of their own, took 23 launches and copies an image kind where this takes
+// four: about 4 us apiece at the small sizes, and 0.92 ms against 0.39 ms of
+// kernels at 6144^2 x 96 layers, 14 M bins.)
+__device__ __forceinline__ uint32_t extraItems(uint32_t c, uint32_t chunk) {
+  return c > chunk ? (c - 1u) / chunk : 0u;
 }
 
-// The work items: {bin, item index within the bin, first record, records} of
-// every item (thread per bin; a split bin writes one entry per item), so that
-// the grid and degrid kernels find an item's records with one load instead of
-// a chain of three.
+// Pass 1: prefixes within the workgroup's kScanBlock bins, and its totals of
+// records, extra items, items and split bins to sums[0 .. 3][block].
 __global__ void __launch_bounds__(kThreads)
-workItemsKernel(const uint32_t* __restrict__ itemStart, const uint32_t* __restrict__ binStart,
-                size_t nbins, uint32_t chunk, uint4* __restrict__ items) {
-  const size_t b = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b >= nbins) return;
-  const uint32_t i0 = itemStart[b], i1 = itemStart[b + 1];
-  if (i0 == i1) return;
-  const uint32_t s0 = binStart[b], s1 = binStart[b + 1];
-  for (uint32_t i = i0; i < i1; ++i) {
-    const uint32_t j = i - i0, start = s0 + j * chunk;
-    items[i] = make_uint4(uint32_t(b), j, start, min(s1 - start, chunk));
+binScanKernel(const uint32_t* __restrict__ counts, size_t nbins, uint32_t chunk,
+              uint32_t* __restrict__ binStart, uint32_t* __restrict__ extraStart,
+              uint32_t* __restrict__ itemStart, uint32_t* __restrict__ sums) {
+  __shared__ uint32_t sh[kThreads / 64];
+  const size_t b0 = size_t(blockIdx.x) * kScanBlock + size_t(threadIdx.x) * kScanItems;
+  uint32_t c[kScanItems];
+  uint32_t r = 0u, e = 0u, n = 0u, s = 0u;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    c[k] = b0 + k < nbins ? counts[b0 + k] : 0u;
+    r += c[k];
+    e += extraItems(c[k], chunk);
+    n += c[k] ? 1u : 0u;
+    s += c[k] > chunk ? 1u : 0u;
+  }
+  uint32_t tr, te, tn, ts;
+  (void)blockExclusiveScan(s, sh, &ts);
+  r = blockExclusiveScan(r, sh, &tr);
+  e = blockExclusiveScan(e, sh, &te);
+  n = blockExclusiveScan(n, sh, &tn);
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    if (b0 + k >= nbins) break;
+    binStart[b0 + k] = r;
+    extraStart[b0 + k] = e;
+    itemStart[b0 + k] = n + e;
+    r += c[k];
+    e += extraItems(c[k], chunk);
+    n += c[k] ? 1u : 0u;
+  }
+  if (threadIdx.x == 0) {
+    sums[blockIdx.x] = tr;
+    sums[gridDim.x + blockIdx.x] = te;
+    sums[2 * size_t(gridDim.x) + blockIdx.x] = tn + te;
+    sums[3 * size_t(gridDim.x) + blockIdx.x] = ts;
   }
 }
 
-// Occupancy bits: bit b of the array is set when bin b holds records
-// (thread per 32-bit word).
+// The workgroups' totals turned into their offsets (one workgroup), the plan's
+// totals to totals[0 .. 3] (records, extra items, items, split bins) and the
+// non-empty bins to *used and *occupied.
 __global__ void __launch_bounds__(kThreads)
-occupancyKernel(const uint32_t* __restrict__ binStart, size_t nbins,
-                uint32_t* __restrict__ occ) {
-  const size_t w = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t b0 = w * 32;
-  if (b0 >= nbins) return;
-  uint32_t bits = 0;
-  for (int j = 0; j < 32 && b0 + j < nbins; ++j)
-    if (binStart[b0 + j + 1] > binStart[b0 + j]) bits |= 1u << j;
-  occ[w] = bits;
+binScanSumsKernel(uint32_t* __restrict__ sums, size_t nblocks,
+                  unsigned long long* __restrict__ totals, unsigned long long* __restrict__ used,
+                  unsigned long long* __restrict__ occupied) {
+  __shared__ uint32_t sh[kThreads / 64];
+  uint32_t total[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t* v = sums + size_t(q) * nblocks;
+    uint32_t carry = 0u;
+    for (size_t b0 = 0; b0 < nblocks; b0 += kScanBlock) {
+      const size_t b = b0 + size_t(threadIdx.x) * kScanItems;
+      uint32_t x[kScanItems], local = 0u, t;
+#pragma unroll
+      for (int k = 0; k < kScanItems; ++k) {
+        x[k] = b + k < nblocks ? v[b + k] : 0u;
+        local += x[k];
+      }
+      uint32_t run = carry + blockExclusiveScan(local, sh, &t);
+#pragma unroll
+      for (int k = 0; k < kScanItems; ++k) {
+        if (b + k < nblocks) v[b + k] = run;
+        run += x[k];
+      }
+      carry += t;
+    }
+    total[q] = carry;
+  }
+  if (threadIdx.x == 0) {
+    for (int q = 0; q < 4; ++q) totals[q] = total[q];
+    *used = total[2] - total[1];
+    *occupied = total[2] - total[1];
+  }
+}
+
+// Pass 2: adds the workgroups' offsets, and per bin sets the scatter cursor
+// (in place of the counts), the occupancy bit (bit b of occ: bin b holds
+// records), the bin's work items {bin, index within the bin, first record,
+// records} -- so that the grid and degrid kernels find an item's records with
+// one load instead of a chain of three -- and lists the split bins.
+__global__ void __launch_bounds__(kThreads)
+binFinishKernel(uint32_t* __restrict__ counts, size_t nbins, uint32_t chunk,
+                uint32_t* __restrict__ binStart, uint32_t* __restrict__ extraStart,
+                uint32_t* __restrict__ itemStart, const uint32_t* __restrict__ sums,
+                const unsigned long long* __restrict__ totals, uint8_t* __restrict__ occ,
+                size_t occBytes, uint4* __restrict__ items, uint32_t* __restrict__ splitBins,
+                uint32_t nSplit) {
+  // bins of many items (the dense uv centre's hold thousands), whose items
+  // the whole workgroup writes: {bin, first item, first record, records}
+  constexpr uint32_t kAlone = 8u, kBig = 64u;
+  __shared__ uint4 big[kBig];
+  __shared__ uint32_t nBig;
+  __shared__ uint32_t sh[kThreads / 64];
+  if (threadIdx.x == 0) nBig = 0u;
+  const uint32_t offR = sums[blockIdx.x], offE = sums[gridDim.x + blockIdx.x],
+                 offI = sums[2 * size_t(gridDim.x) + blockIdx.x];
+  const size_t b0 = size_t(blockIdx.x) * kScanBlock + size_t(threadIdx.x) * kScanItems;
+  uint32_t cnt[kScanItems], splits = 0u, blockSplits;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    cnt[k] = b0 + k < nbins ? counts[b0 + k] : 0u;
+    splits += cnt[k] > chunk ? 1u : 0u;
+  }
+  uint32_t split = sums[3 * size_t(gridDim.x) + blockIdx.x] +
+                   blockExclusiveScan(splits, sh, &blockSplits);
+  uint32_t bits = 0u;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    const size_t b = b0 + k;
+    if (b >= nbins) break;
+    const uint32_t c = cnt[k];
+    const uint32_t r = binStart[b] + offR, i0 = itemStart[b] + offI;
+    binStart[b] = r;
+    extraStart[b] += offE;
+    itemStart[b] = i0;
+    counts[b] = r;
+    if (c == 0u) continue;
+    bits |= 1u << k;
+    const uint32_t n = 1u + extraItems(c, chunk);
+    const uint32_t at = n > kAlone ? atomicAdd(&nBig, 1u) : kBig;
+    if (at < kBig)
+      big[at] = make_uint4(uint32_t(b), i0, r, c);
+    else
+      for (uint32_t j = 0; j < n; ++j)
+        items[i0 + j] = make_uint4(uint32_t(b), j, r + j * chunk, min(c - j * chunk, chunk));
+    if (n > 1u) {
+      if (split < nSplit) splitBins[split] = uint32_t(b);
+      ++split;
+    }
+  }
+  if ((b0 >> 3) < occBytes) occ[b0 >> 3] = uint8_t(bits);
+  __syncthreads();
+  for (uint32_t q = 0; q < min(nBig, kBig); ++q) {
+    const uint4 d = big[q];
+    const uint32_t n = 1u + extraItems(d.w, chunk);
+    for (uint32_t j = threadIdx.x; j < n; j += kThreads)
+      items[d.y + j] = make_uint4(d.x, j, d.z + j * chunk, min(d.w - j * chunk, chunk));
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    binStart[nbins] = uint32_t(totals[0]);
+    extraStart[nbins] = uint32_t(totals[1]);
+    itemStart[nbins] = uint32_t(totals[2]);
+  }
+}
+
+// The number of set bits among the workgroup's threads' words, added to *out
+// by one atomic (atomics on one address return about every 13 ns).
+__device__ __forceinline__ void addBits(uint32_t bits, unsigned long long* out) {
+  __shared__ uint32_t sum;
+  if (threadIdx.x == 0) sum = 0u;
+  __syncthreads();
+  int v = __popc(bits);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if ((threadIdx.x & 63) == 0 && v) atomicAdd(&sum, uint32_t(v));
+  __syncthreads();
+  if (threadIdx.x == 0 && sum) atomicAdd(out, (unsigned long long)sum);
 }
 
 // Row bits: bit (layer * tilesY + ty) is set when some tile of that tile row
 // holds records (thread per bit, packed by wave ballots).
 __global__ void __launch_bounds__(kThreads)
 rowLiveKernel(const uint32_t* __restrict__ occ, size_t nrows, int tilesX,
-              uint32_t* __restrict__ rowLive) {
+              uint32_t* __restrict__ rowLive, unsigned long long* __restrict__ total) {
   const size_t r = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  bool live = false;
+  uint32_t any = 0u;
   if (r < nrows) {
-    const size_t b0 = r * size_t(tilesX);
-    for (int t = 0; t < tilesX && !live; ++t) {
-      const size_t b = b0 + t;
-      live = (occ[b >> 5] >> (b & 31)) & 1u;
+    // bits [b0, b1) of the occupancy, word by word
+    const size_t b0 = r * size_t(tilesX), b1 = b0 + size_t(tilesX);
+    for (size_t w = b0 >> 5; w <= (b1 - 1) >> 5; ++w) {
+      uint32_t v = occ[w];
+      if (w == b0 >> 5) v &= ~0u << (b0 & 31);
+      if (w == (b1 - 1) >> 5) v &= ~0u >> (31 - ((b1 - 1) & 31));
+      any |= v;
     }
   }
-  const unsigned long long m = __ballot(live);
+  const unsigned long long m = __ballot(any != 0u);
   const size_t w0 = (r & ~size_t(63)) >> 5;  // first word of this wave's 64 bits
   const int lane = threadIdx.x & 63;
   if (lane == 0 && w0 < (nrows + 31) / 32) rowLive[w0] = uint32_t(m);
   if (lane == 32 && w0 + 1 < (nrows + 31) / 32) rowLive[w0 + 1] = uint32_t(m >> 32);
-}
-
-// Adds the set bits of a bit array to *out (thread per 32-bit word).
-__global__ void __launch_bounds__(kThreads)
-popcountKernel(const uint32_t* __restrict__ bits, size_t words,
-               unsigned long long* __restrict__ out) {
-  const size_t w = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int c = w < words ? __popc(bits[w]) : 0;
-  // wave sum, one atomic per wave
-  int v = c;
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0 && v) atomicAdd(out, (unsigned long long)v);
+  addBits(any ? 1u : 0u, total);
 }
 
 // Column bits: bit (layer * tilesX + tx) is set when some tile row of that
@@ -595,21 +734,24 @@ popcountKernel(const uint32_t* __restrict__ bits, size_t words,
 // forward rows pass writes.
 __global__ void __launch_bounds__(kThreads)
 liveColumnsKernel(const uint32_t* __restrict__ bits, size_t ncols, int tilesX, int tilesY,
-                  uint32_t* __restrict__ colBits) {
+                  uint32_t* __restrict__ colBits, unsigned long long* __restrict__ total) {
   const size_t c = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  bool live = false;
+  uint32_t live = 0u;
   if (c < ncols) {
     const size_t layer = c / size_t(tilesX), tx = c - layer * size_t(tilesX);
-    for (int ty = 0; ty < tilesY && !live; ++ty) {
+    // (no early exit: the loads are independent)
+#pragma unroll 8
+    for (int ty = 0; ty < tilesY; ++ty) {
       const size_t b = (layer * size_t(tilesY) + size_t(ty)) * size_t(tilesX) + tx;
-      live = (bits[b >> 5] >> (b & 31)) & 1u;
+      live |= (bits[b >> 5] >> (b & 31)) & 1u;
     }
   }
-  const unsigned long long m = __ballot(live);
+  const unsigned long long m = __ballot(live != 0u);
   const size_t w0 = (c & ~size_t(63)) >> 5;  // first word of this wave's 64 bits
   const int lane = threadIdx.x & 63;
   if (lane == 0 && w0 < (ncols + 31) / 32) colBits[w0] = uint32_t(m);
   if (lane == 32 && w0 + 1 < (ncols + 31) / 32) colBits[w0 + 1] = uint32_t(m >> 32);
+  addBits(live, total);
 }
 
 // Need bits: tile (tx, ty) of a layer is read by the degridding subgrids of
@@ -618,10 +760,9 @@ liveColumnsKernel(const uint32_t* __restrict__ bits, size_t ncols, int tilesX, i
 // wrapping round the grid). Thread per 32-bit word.
 __global__ void __launch_bounds__(kThreads)
 needKernel(const uint32_t* __restrict__ occ, size_t nbins, int tilesX, int tilesY,
-           uint32_t* __restrict__ need) {
+           uint32_t* __restrict__ need, unsigned long long* __restrict__ total) {
   const size_t w = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t b0 = w * 32;
-  if (b0 >= nbins) return;
   const size_t perLayer = size_t(tilesX) * tilesY;
   auto bit = [&](size_t b) { return (occ[b >> 5] >> (b & 31)) & 1u; };
   uint32_t bits = 0;
@@ -636,7 +777,8 @@ needKernel(const uint32_t* __restrict__ occ, size_t nbins, int tilesX, int tiles
                        bit(layerBase + size_t(py) * tilesX + px);
     bits |= v << j;
   }
-  need[w] = bits;
+  if (b0 < nbins) need[w] = bits;
+  addBits(bits, total);
 }
 
 // One work item of a pass: bin, item index within the bin (0 = the item
@@ -645,21 +787,6 @@ needKernel(const uint32_t* __restrict__ occ, size_t nbins, int tilesX, int tiles
 struct WorkItem {
   uint32_t bin, j, start, count;
 };
-
-// Largest b in [lo, hi) with offs[b] <= v, for nondecreasing offs with
-// offs[lo] <= v < offs[hi]: the bin that owns entry v (bins owning no entry
-// are skipped because the next bin has the same offset).
-__device__ __forceinline__ uint32_t ownerOf(const uint32_t* __restrict__ offs, uint32_t lo,
-                                            uint32_t hi, uint32_t v) {
-  while (hi - lo > 1u) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (offs[mid] <= v)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
-}
 
 __device__ __forceinline__ WorkItem workItem(const uint4* __restrict__ items, uint32_t i) {
   const uint4 d = items[i];
@@ -673,33 +800,12 @@ __device__ __forceinline__ uint32_t passItems(uint32_t binLo, uint32_t binHi,
 
 
 // --------------------------------------------------------- exclusive scan
-constexpr int kScanItems = 8;
-constexpr int kScanBlock = kThreads * kScanItems;  // 2048 values per block
-
-__device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v,
-                                                       uint32_t* sh,
-                                                       uint32_t* total) {
-  const int tid = threadIdx.x;
-  sh[tid] = v;
-  __syncthreads();
-  for (int off = 1; off < kThreads; off <<= 1) {
-    uint32_t t = (tid >= off) ? sh[tid - off] : 0u;
-    __syncthreads();
-    sh[tid] += t;
-    __syncthreads();
-  }
-  const uint32_t incl = sh[tid];
-  *total = sh[kThreads - 1];
-  __syncthreads();
-  return incl - v;
-}
-
 // out[i] = sum_{j<i} in[j] within each block of kScanBlock values; block
-// totals to blockSums.
+// totals to blockSums (a single workgroup writes the total to out[n] too).
 __global__ void __launch_bounds__(kThreads)
 scanBlocksKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                  size_t n, uint32_t* __restrict__ blockSums) {
-  __shared__ uint32_t sh[kThreads];
+  __shared__ uint32_t sh[kThreads / 64];
   const size_t base = size_t(blockIdx.x) * kScanBlock + size_t(threadIdx.x) * kScanItems;
   uint32_t vals[kScanItems];
   uint32_t local = 0;
@@ -717,20 +823,20 @@ scanBlocksKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
     if (i < n) out[i] = run;
     run += vals[k];
   }
-  if (threadIdx.x == 0) blockSums[blockIdx.x] = total;
+  if (threadIdx.x == 0) {
+    blockSums[blockIdx.x] = total;
+    if (gridDim.x == 1) out[n] = total;
+  }
 }
 
-__global__ void scanAddKernel(uint32_t* __restrict__ out, size_t n,
-                              const uint32_t* __restrict__ blockOffsets) {
+// Adds the blocks' offsets; out[n] = the total.
+__global__ void scanAddKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                              size_t n, const uint32_t* __restrict__ blockOffsets) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) out[i] += blockOffsets[i / kScanBlock];
-}
-
-// out[n] = total is written as well (out has n + 1 entries).
-__global__ void scanTotalKernel(const uint32_t* __restrict__ in,
-                                uint32_t* __restrict__ out, size_t n) {
-  if (threadIdx.x == 0 && blockIdx.x == 0)
-    out[n] = (n > 0) ? out[n - 1] + in[n - 1] : 0u;
+  if (i >= n) return;
+  const uint32_t v = out[i] + blockOffsets[i / kScanBlock];
+  out[i] = v;
+  if (i == n - 1) out[n] = v + in[i];
 }
 
 // ------------------------------------------------------------- grid (LDS)
@@ -2110,32 +2216,31 @@ degridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
 constexpr int kReduceParts = 4;  // threads summing one cell's partial tiles
 
 // Adds the partial tiles of the extra items of every split bin of a pass to
-// the layer, in a fixed summation order. Task (e, group): if e is the first
-// extra item of its bin, the workgroup sums that bin's partial tiles for one
-// group of 256 / kReduceParts cells, kReduceParts threads per cell
-// (coalesced over the cells of each partial tile): the dense uv centre's
-// bins hold thousands of extra items, and one thread per cell left their
-// sums latency-bound.
+// the layer, in a fixed summation order. Task (split bin, group): the
+// workgroup sums that bin's partial tiles for one group of 256 / kReduceParts
+// cells, kReduceParts threads per cell (coalesced over the cells of each
+// partial tile): the dense uv centre's bins hold thousands of extra items, and
+// one thread per cell left their sums latency-bound.
 template <int NIMG>
 __global__ void __launch_bounds__(kThreads)
 reducePartialsKernel(GridArgs a, const uint32_t* __restrict__ extraStart,
+                     const uint32_t* __restrict__ splitBins, uint32_t nSplit,
                      const float2* __restrict__ partials, float2* __restrict__ layers) {
   __shared__ float2 red[kReduceParts][kThreads / kReduceParts];
   const uint32_t binLo = uint32_t(a.layerLo) * uint32_t(a.tilesPerLayer);
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
-  const uint32_t eLo = extraStart[binLo], eHi = extraStart[binHi];
   const int T = a.ga.tileSize, T2 = T * T;
   constexpr int kCells = kThreads / kReduceParts;  // cells per task
   const uint32_t groups = uint32_t((T2 + kCells - 1) / kCells);
   const size_t HW = size_t(a.ga.W) * a.ga.H;
-  const size_t tasks = size_t(eHi - eLo) * groups;
+  const size_t tasks = size_t(nSplit) * groups;
   const int part = int(threadIdx.x) / kCells, cl = int(threadIdx.x) - part * kCells;
   for (size_t task = blockIdx.x; task < tasks; task += gridDim.x) {
-    const uint32_t e = eLo + uint32_t(task / groups);
-    const uint32_t grp = uint32_t(task - size_t(e - eLo) * groups);
-    const uint32_t bin = ownerOf(extraStart, binLo, binHi, e);
+    const uint32_t sb = uint32_t(task / groups);
+    const uint32_t grp = uint32_t(task - size_t(sb) * groups);
+    const uint32_t bin = splitBins[sb];
+    if (bin < binLo || bin >= binHi) continue;  // of another pass (workgroup-uniform)
     const uint32_t first = extraStart[bin];
-    if (e != first) continue;  // another task of the bin does the work (workgroup-uniform)
     const int c = int(grp) * kCells + cl;
     const bool valid = c < T2;
     const uint32_t nEx = extraStart[bin + 1] - first;
@@ -2598,11 +2703,10 @@ hws_status exclusiveScan(hws_gridder* g, const uint32_t* in, uint32_t* out,
   HWS_TRY(checkHip(g, hipGetLastError(), "scan blocks"));
   if (nblocks > 1) {
     HWS_TRY(exclusiveScan(g, sums, offs, nblocks, scratch + 2 * (nblocks + 1)));
-    hipLaunchKernelGGL(scanAddKernel, dim3(blocksFor(n)), dim3(kThreads), 0, g->stream, out, n, offs);
+    hipLaunchKernelGGL(scanAddKernel, dim3(blocksFor(n)), dim3(kThreads), 0, g->stream, in, out, n, offs);
     HWS_TRY(checkHip(g, hipGetLastError(), "scan add"));
   }
-  hipLaunchKernelGGL(scanTotalKernel, dim3(1), dim3(64), 0, g->stream, in, out, n);
-  return checkHip(g, hipGetLastError(), "scan total");
+  return HWS_OK;
 }
 
 namespace {
@@ -2650,6 +2754,8 @@ ImgArgs imgArgs(const hws_gridder* g, int pass) {
   a.fresh = 0;
   return a;
 }
+
+constexpr size_t kUnsortedRows = 4096;  // binned without the row sort up to here
 
 // The matrix-core grid kernel covers 16 x 16 tiles with the padded table.
 bool mfmaKernelUsable(const hws_gridder* g) {
@@ -2771,8 +2877,14 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
   pl.nbins = tpl * size_t(g->nW);
   if (pl.nbins >= 0xFFFFFFFFull)
     return setLastError(g, HWS_ERR_UNSUPPORTED, "too many (layer, tile) bins");
-  HWS_TRY(ensureAlloc(g, pl.scanScratch, pl.scanScratchCapacity, scanScratchSize(pl.nbins),
+  const size_t scanBlocks = (pl.nbins + kScanBlock - 1) / kScanBlock;
+  // (both image kinds are counted before either is laid out)
+  HWS_TRY(ensureAlloc(g, pl.scanScratch, pl.scanScratchCapacity, 2 * 4 * scanBlocks,
                       "plan scan scratch"));
+  if (!pl.hostCounters)
+    HWS_TRY(checkHip(g, hipHostMalloc(reinterpret_cast<void**>(&pl.hostCounters),
+                                      kPlanCounters * sizeof(unsigned long long)),
+                     "plan counters"));
   if (!pl.counters)
     HWS_TRY(checkHip(g, hipMalloc(&pl.counters, kPlanCounters * sizeof(unsigned long long)),
                      "plan counters"));
@@ -2795,16 +2907,27 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
                       "row order"));
   if (n > 0) {
     hipLaunchKernelGGL(rowKeyKernel, dim3(blocksFor(nrow)), dim3(kThreads), 0, g->stream, dUvw,
-                       dWl, nrow, int(nchan), ga, layerMap(g, keyKind), pl.rowKeys, pl.rowOrder);
+                       dWl, nrow, int(nchan), ga, layerMap(g, keyKind), uint32_t(pl.nbins),
+                       pl.rowKeys, pl.rowOrder);
     HWS_TRY(checkHip(g, hipGetLastError(), "row key launch"));
-    HWS_TRY(sortRows(g, pl.rowKeys, pl.rowKeysAlt, pl.rowOrder, pl.rowOrderAlt, nrow));
+    // (a few thousand rows are binned as they come: their sort takes six to
+    // twelve launches, about 60 us, and saves less in the binning's atomics:
+    // 2016 rows x 16 channels, the scatter takes 12 us either way)
+    if (nrow > kUnsortedRows) {
+      int keyBits = 1;  // keys run from 0 to nbins
+      while (keyBits < 32 && (size_t(1) << keyBits) <= pl.nbins) ++keyBits;
+      HWS_TRY(sortRows(g, pl.rowKeys, pl.rowKeysAlt, pl.rowOrder, pl.rowOrderAlt, nrow, keyBits));
+    }
   }
   // row groups of PER * 256 samples, visited with a stride coprime to their
   // number: the count pass takes 16 samples per thread and group, the
   // scatter (which keeps its records in registers until the group's
   // positions are known) 2 (measured best of 2-16 and 1-4 at the 4096^2
-  // benchmark)
-  constexpr int countPer = 16, scatterPer = 2;
+  // benchmark); a count of few samples takes 4 or 1, so that its groups fill
+  // the chip (32 k samples: 38 us with 16, 7 with 1)
+  constexpr int scatterPer = 2;
+  const size_t countGroups = size_t(persistentBlocks(g, 2)) * kThreads;
+  const int countPer = n >= countGroups * 16 ? 16 : n >= countGroups * 4 ? 4 : 1;
   auto groupsOf = [&](int per, uint32_t& ngroups, uint32_t& step, unsigned& blocks) {
     const size_t gs = size_t(per) * kThreads;
     ngroups = uint32_t((n + gs - 1) / gs);
@@ -2846,82 +2969,77 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
 #define HWS_COUNT(P)                                                                      \
   hipLaunchKernelGGL((binKernel<false, false, P>), dim3(cBlocks), dim3(kThreads), 0, g->stream, \
                      dUvw, dWl, pl.rowOrder, nrow, int(nchan), cGroups, cStep, ga, ka)
-      HWS_COUNT(countPer);
+      if (countPer == 16)
+        HWS_COUNT(16);
+      else if (countPer == 4)
+        HWS_COUNT(4);
+      else
+        HWS_COUNT(1);
 #undef HWS_COUNT
       HWS_TRY(checkHip(g, hipGetLastError(), "bin count launch"));
     }
-    HWS_TRY(exclusiveScan(g, kp.counts, kp.binStart, pl.nbins, pl.scanScratch));
-    // work items: the counts array is free until the scatter cursor is set
-    hipLaunchKernelGGL(extraItemsKernel, dim3(blocksFor(pl.nbins)), dim3(kThreads), 0,
-                       g->stream, kp.binStart, pl.nbins, pl.chunk, kp.counts,
-                       pl.counters + 6 + kind);
-    HWS_TRY(checkHip(g, hipGetLastError(), "work item launch"));
-    HWS_TRY(exclusiveScan(g, kp.counts, kp.extraStart, pl.nbins, pl.scanScratch));
-    hipLaunchKernelGGL(binItemsKernel, dim3(blocksFor(pl.nbins)), dim3(kThreads), 0, g->stream,
-                       kp.binStart, kp.extraStart, pl.nbins, kp.counts);
-    HWS_TRY(checkHip(g, hipGetLastError(), "work item launch"));
-    HWS_TRY(exclusiveScan(g, kp.counts, kp.itemStart, pl.nbins, pl.scanScratch));
-    // the record and item totals size the sorted array and partials
-    uint32_t totals[3] = {0, 0, 0};
-    unsigned long long placed[3] = {0ull, 0ull, 0ull};
-    HWS_TRY(checkHip(g, hipMemcpyAsync(placed, pl.counters + 3 * kind, sizeof(placed),
-                                       hipMemcpyDeviceToHost, g->stream), "sample counts"));
-    HWS_TRY(checkHip(g, hipMemcpyAsync(&totals[0], kp.binStart + pl.nbins, sizeof(uint32_t),
-                                       hipMemcpyDeviceToHost, g->stream), "record total"));
-    HWS_TRY(checkHip(g, hipMemcpyAsync(&totals[1], kp.extraStart + pl.nbins, sizeof(uint32_t),
-                                       hipMemcpyDeviceToHost, g->stream), "item total"));
-    HWS_TRY(checkHip(g, hipMemcpyAsync(&totals[2], kp.itemStart + pl.nbins, sizeof(uint32_t),
-                                       hipMemcpyDeviceToHost, g->stream), "item total"));
-    HWS_TRY(checkHip(g, hipStreamSynchronize(g->stream), "plan totals"));
-    const uint32_t total = totals[0];
+    uint32_t* sums = pl.scanScratch + size_t(kind) * 4 * scanBlocks;
+    hipLaunchKernelGGL(binScanKernel, dim3(unsigned(scanBlocks)), dim3(kThreads), 0, g->stream,
+                       kp.counts, pl.nbins, pl.chunk, kp.binStart, kp.extraStart, kp.itemStart,
+                       sums);
+    hipLaunchKernelGGL(binScanSumsKernel, dim3(1), dim3(kThreads), 0, g->stream, sums,
+                       scanBlocks, pl.counters + 20 + 4 * kind, pl.counters + 6 + kind,
+                       pl.counters + 8 + kind);
+    HWS_TRY(checkHip(g, hipGetLastError(), "bin scan launch"));
+  }
+  // the record and item totals size the sorted arrays and partials
+  HWS_TRY(checkHip(g, hipMemcpyAsync(pl.hostCounters, pl.counters,
+                                     kPlanCounters * sizeof(unsigned long long),
+                                     hipMemcpyDeviceToHost, g->stream), "plan totals"));
+  HWS_TRY(checkHip(g, hipStreamSynchronize(g->stream), "plan totals"));
+  for (int kind = 0; kind < 2; ++kind) {
+    KindPlan& kp = pl.kinds[kind];
+    if (!kp.active) continue;
+    const unsigned long long* placed = pl.hostCounters + 3 * kind;
+    const unsigned long long* totals = pl.hostCounters + 20 + 4 * kind;
+    const uint32_t total = uint32_t(totals[0]);
     kp.nSkipped = placed[1] + placed[2];
     HWS_TRY(ensureAlloc(g, kp.skipped, kp.skippedCapacity,
                         std::max<size_t>(size_t(kp.nSkipped), 1), "plan skipped samples"));
     kp.nItems = total;
     kp.nExtra = totals[1];
     kp.nWorkItems = totals[2];
+    kp.nSplit = totals[3];
     HWS_TRY(ensureAlloc(g, kp.items, kp.workItemCapacity, size_t(kp.nWorkItems),
                         "plan work items"));
+    HWS_TRY(ensureAlloc(g, kp.splitBins, kp.splitCapacity, size_t(kp.nSplit),
+                        "plan split bins"));
     const size_t occWords = (pl.nbins + 31) / 32;
     HWS_TRY(ensureAlloc(g, kp.occ, kp.occCapacity, occWords, "plan occupancy"));
-    hipLaunchKernelGGL(occupancyKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
-                       kp.binStart, pl.nbins, kp.occ);
-    HWS_TRY(checkHip(g, hipGetLastError(), "occupancy launch"));
     const size_t nrowsBits = pl.nbins / size_t(pl.tilesX);
     const size_t rowWords = (nrowsBits + 31) / 32;
     HWS_TRY(ensureAlloc(g, kp.rowLive, kp.rowLiveCapacity, rowWords, "plan row bits"));
-    hipLaunchKernelGGL(rowLiveKernel, dim3(blocksFor(nrowsBits)), dim3(kThreads), 0, g->stream,
-                       kp.occ, nrowsBits, pl.tilesX, kp.rowLive);
-    HWS_TRY(checkHip(g, hipGetLastError(), "row bits launch"));
     HWS_TRY(ensureAlloc(g, kp.need, kp.needCapacity, occWords, "plan need bits"));
-    hipLaunchKernelGGL(needKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
-                       kp.occ, pl.nbins, pl.tilesX, pl.tilesY, kp.need);
-    HWS_TRY(checkHip(g, hipGetLastError(), "need launch"));
-    hipLaunchKernelGGL(popcountKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
-                       kp.occ, occWords, pl.counters + 8 + kind);
-    hipLaunchKernelGGL(popcountKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
-                       kp.need, occWords, pl.counters + 10 + kind);
-    hipLaunchKernelGGL(popcountKernel, dim3(blocksFor(rowWords)), dim3(kThreads), 0, g->stream,
-                       kp.rowLive, rowWords, pl.counters + 14 + kind);
     const size_t ncolsBits = pl.nbins / size_t(pl.tilesY);
     const size_t colWords = (ncolsBits + 31) / 32;
     HWS_TRY(ensureAlloc(g, kp.colNeed, kp.colNeedCapacity, colWords, "plan column bits"));
+    // (sets the scatter cursor in place of the counts)
+    hipLaunchKernelGGL(binFinishKernel, dim3(unsigned(scanBlocks)), dim3(kThreads), 0, g->stream,
+                       kp.counts, pl.nbins, pl.chunk, kp.binStart, kp.extraStart, kp.itemStart,
+                       pl.scanScratch + size_t(kind) * 4 * scanBlocks,
+                       pl.counters + 20 + 4 * kind, reinterpret_cast<uint8_t*>(kp.occ),
+                       occWords * 4, kp.items, kp.splitBins, uint32_t(kp.nSplit));
+    HWS_TRY(checkHip(g, hipGetLastError(), "bin offsets launch"));
+    hipLaunchKernelGGL(rowLiveKernel, dim3(blocksFor(nrowsBits)), dim3(kThreads), 0, g->stream,
+                       kp.occ, nrowsBits, pl.tilesX, kp.rowLive, pl.counters + 14 + kind);
+    hipLaunchKernelGGL(needKernel, dim3(blocksFor(occWords)), dim3(kThreads), 0, g->stream,
+                       kp.occ, pl.nbins, pl.tilesX, pl.tilesY, kp.need, pl.counters + 10 + kind);
     hipLaunchKernelGGL(liveColumnsKernel, dim3(blocksFor(ncolsBits)), dim3(kThreads), 0,
-                       g->stream, kp.need, ncolsBits, pl.tilesX, pl.tilesY, kp.colNeed);
-    hipLaunchKernelGGL(popcountKernel, dim3(blocksFor(colWords)), dim3(kThreads), 0, g->stream,
-                       kp.colNeed, colWords, pl.counters + 16 + kind);
-    HWS_TRY(checkHip(g, hipGetLastError(), "tile count launch"));
-    hipLaunchKernelGGL(workItemsKernel, dim3(blocksFor(pl.nbins)), dim3(kThreads), 0, g->stream,
-                       kp.itemStart, kp.binStart, pl.nbins, pl.chunk, kp.items);
-    HWS_TRY(checkHip(g, hipGetLastError(), "work item launch"));
+                       g->stream, kp.need, ncolsBits, pl.tilesX, pl.tilesY, kp.colNeed,
+                       pl.counters + 16 + kind);
+    HWS_TRY(checkHip(g, hipGetLastError(), "tile bits launch"));
     HWS_TRY(ensureAlloc(g, kp.recSorted, kp.capacity, size_t(total), "plan sorted records"));
     if (kp.nExtra)
       HWS_TRY(ensureAlloc(g, kp.partials, kp.partialCapacity,
                           size_t(kp.nExtra) * kp.nImg * pl.tileSize * pl.tileSize,
                           "plan partial tiles"));
-    // cursor = bin offsets
-    HWS_TRY(checkHip(g, hipMemcpyAsync(kp.counts, kp.binStart, pl.nbins * sizeof(uint32_t),
-                                       hipMemcpyDeviceToDevice, g->stream), "cursor copy"));
+    KindArgs ka{layerMap(g, kind), kp.counts, nullptr, nullptr, pl.counters + 3 * kind,
+                nullptr, 0u, nullptr, 0u, pl.counters + 18 + kind};
     ka.cursor = kp.counts;
     ka.recSorted = kp.recSorted;
     ka.nRecords = total;
@@ -2962,9 +3080,10 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
       if (kp.recSorted != r0) std::swap(kp.capacity, kp.altCapacity);
     }
   }
-  unsigned long long c[kPlanCounters] = {};
-  HWS_TRY(checkHip(g, hipMemcpyAsync(c, pl.counters, sizeof(c), hipMemcpyDeviceToHost,
-                                     g->stream), "plan check"));
+  const unsigned long long* c = pl.hostCounters;
+  HWS_TRY(checkHip(g, hipMemcpyAsync(pl.hostCounters, pl.counters,
+                                     kPlanCounters * sizeof(unsigned long long),
+                                     hipMemcpyDeviceToHost, g->stream), "plan check"));
   HWS_TRY(checkHip(g, hipStreamSynchronize(g->stream), "plan check"));
   bool listed = true;
   for (int kind = 0; kind < 2; ++kind)
@@ -3181,12 +3300,12 @@ hws_status gridBinned(hws_gridder* g, const float* dVis, int pass, bool accumula
       if (kp.nExtra) {
         const uint64_t cells = kThreads / kReduceParts;
         const uint64_t groups = (uint64_t(pl.tileSize) * pl.tileSize + cells - 1) / cells;
-        const unsigned rblocks = unsigned(std::min<uint64_t>(kp.nExtra * groups, 65536));
+        const unsigned rblocks = unsigned(std::min<uint64_t>(kp.nSplit * groups, 65536));
         switch (n) {
 #define HWS_REDUCE_CASE(N)                                                                    \
   case N:                                                                                     \
     hipLaunchKernelGGL(reducePartialsKernel<N>, dim3(rblocks), dim3(kThreads), 0, g->stream,   \
-                       a, kp.extraStart, kp.partials, layers);                                \
+                       a, kp.extraStart, kp.splitBins, uint32_t(kp.nSplit), kp.partials, layers);                                \
     break;
           HWS_REDUCE_CASE(1)
           HWS_REDUCE_CASE(2)
@@ -3589,18 +3708,26 @@ weightSumsKernel(const double* __restrict__ uvw, const double* __restrict__ wl, 
     }
 }
 
-// Sums the block partials in block order (one thread per image and counter).
-__global__ void weightSumsFinalKernel(const double* __restrict__ partials, int nblocks, int nImg,
-                                      double* __restrict__ sums) {
-  const int t = threadIdx.x;
-  if (t >= nImg * 4) return;
-  const int i = t / 4, q = t - i * 4;
-  double r = 0.0;
-  for (int b = 0; b < nblocks; ++b) {
-    const double v = partials[(size_t(b) * kMaxImages + i) * 4 + q];
-    r = q == 2 ? fmax(r, v) : r + v;
+constexpr int kSumBlocks = 1024;  // workgroups (partial sums) of the weight sums
+
+// Sums the block partials, a workgroup of 64 lanes per image and counter: a
+// lane sums every 64th in order, the lanes' sums are added by a fixed tree.
+// (One thread for all 1024 waited out as many dependent loads: 250-390 us.)
+__global__ void __launch_bounds__(64)
+weightSumsFinalKernel(const double* __restrict__ partials, double* __restrict__ sums) {
+  const int t = blockIdx.x, q = t & 3;
+  double v[kSumBlocks / 64];
+#pragma unroll
+  for (int k = 0; k < kSumBlocks / 64; ++k)
+    v[k] = partials[size_t(k * 64 + int(threadIdx.x)) * (kMaxImages * 4) + t];
+  double r = v[0];
+#pragma unroll
+  for (int k = 1; k < kSumBlocks / 64; ++k) r = q == 2 ? fmax(r, v[k]) : r + v[k];
+  for (int o = 32; o > 0; o >>= 1) {
+    const double x = __shfl_xor(r, o);
+    r = q == 2 ? fmax(r, x) : r + x;
   }
-  sums[i * 4 + q] = r;
+  if (threadIdx.x == 0) sums[t] = r;
 }
 
 }  // namespace
@@ -3614,7 +3741,7 @@ hws_status planWeights(hws_gridder* g) {
   if (!g->dWeightSums)
     HWS_TRY(checkHip(g, hipMalloc(&g->dWeightSums, kMaxImages * 4 * sizeof(double)),
                      "weight sums"));
-  const int nblocks = 1024;
+  constexpr int nblocks = kSumBlocks;
   if (g->weightPartialCapacity < size_t(nblocks) * kMaxImages * 4) {
     if (g->dWeightPartials) (void)hipFree(g->dWeightPartials);
     g->dWeightPartials = nullptr;
@@ -3651,8 +3778,8 @@ hws_status planWeights(hws_gridder* g) {
       return setLastError(g, HWS_ERR_UNSUPPORTED, "images per context");
   }
   HWS_TRY(checkHip(g, hipGetLastError(), "weight sums launch"));
-  hipLaunchKernelGGL(weightSumsFinalKernel, dim3(1), dim3(64), 0, g->stream,
-                     g->dWeightPartials, nblocks, g->nImg, g->dWeightSums);
+  hipLaunchKernelGGL(weightSumsFinalKernel, dim3(unsigned(g->nImg * 4)), dim3(64), 0, g->stream,
+                     g->dWeightPartials, g->dWeightSums);
   HWS_TRY(checkHip(g, hipGetLastError(), "weight sums launch"));
   pl.weighted = true;
   g->weightSumsValid = true;

@@ -149,8 +149,8 @@ hws_status sortRecords(hws_gridder* g, uint32_t*& keys, uint32_t*& keysAlt, uint
 }
 
 hws_status sortRows(hws_gridder* g, uint32_t*& keys, uint32_t*& keysAlt, uint32_t*& rows,
-                    uint32_t*& rowsAlt, size_t n) {
-  return radixSort(g, keys, keysAlt, rows, rowsAlt, n, 32, "row sort");
+                    uint32_t*& rowsAlt, size_t n, int endBit) {
+  return radixSort(g, keys, keysAlt, rows, rowsAlt, n, endBit, "row sort");
 }
 
 }  // namespace hws
