@@ -408,7 +408,7 @@ constexpr uint32_t kOffsetOutOfRange = 0xFFFFFFF0u;
 
 // Lines (rows or columns) per workgroup, threads and LDS of the transforms.
 unsigned long long packRadices(const FftPlan& plan);
-int threadsFor(const FftPlan& plan, int nfft);
+int threadsFor(const FftPlan& plan, int nfft, bool close = false);
 
 // hws_fft_fused.hip: the fused power-of-two kernels; false where the size has
 // none.
