@@ -478,7 +478,6 @@ void hws_destroy(hws_gridder* g) {
   Plan& pl = g->plan;
   freeDev(pl.scanScratch);
   freeDev(pl.counters);
-  if (pl.hostCounters) (void)hipHostFree(pl.hostCounters);
   freeDev(pl.queue);
   freeDev(pl.rot);
   freeDev(pl.cw);

@@ -329,7 +329,7 @@ struct Plan {
   // gridded, [20 + 4 kind + {0: records, 1: extra items, 2: items, 3: split
   // bins}]
   unsigned long long* counters = nullptr;
-  unsigned long long* hostCounters = nullptr;  // pinned copy
+  unsigned long long hostCounters[kPlanCounters] = {};  // their host copy
   uint32_t* queue = nullptr;  // work-queue counters of the running grid launch
   // rotating contexts: the gridding phase-centre phasor of every sample
   float2* rot = nullptr;
@@ -433,8 +433,8 @@ struct hws_gridder {
   // the mixed precision grids with the FP32 matrix-core kernel
   // (HWS_NO_F16_MFMA=1)
   bool noF16Mfma = false;
-  // degridding workgroups per CU (HWS_DEGRID_BLOCKS_PER_CU)
-  int degridBlocksPerCu = 5;
+  // degridding workgroups per CU (HWS_DEGRID_BLOCKS_PER_CU; 0: by images)
+  int degridBlocksPerCu = 0;
   // lines (rows or columns) per workgroup of the blocked runtime-radix
   // transforms (HWS_FFT_LINES = 1, 2 or 4; 0: chosen by size)
   int fftLines = 0;

@@ -2024,15 +2024,13 @@ template <int NIMG, int KK>
 __device__ __forceinline__ void degridRecord(const GridArgs& a, uint2 rec,
                                              const float* __restrict__ kt,
                                              const float2* __restrict__ sub, int sg,
-                                             const double* __restrict__ uvw,
-                                             const double* __restrict__ wl,
-                                             float2* __restrict__ out) {
+                                             uint32_t byOS, float2* __restrict__ out) {
   const int K = KK ? KK : a.ga.K, OS = a.ga.OS;
   const uint32_t idx = rec.x & 0x3FFFFFFFu;
   const bool conj = (rec.x >> 31) != 0;
   const int xo = int(rec.y & 63u) - (K - 1), yo = int((rec.y >> 6) & 63u) - (K - 1);
   const int kk = int(rec.y >> 12);
-  const int ky = kk / OS, kx = kk - ky * OS;
+  const int ky = kernelRow(kk, byOS), kx = kk - ky * OS;
   float2 acc[NIMG];
 #pragma unroll
   for (int gi = 0; gi < NIMG; ++gi) acc[gi] = make_float2(0.0f, 0.0f);
@@ -2107,13 +2105,10 @@ struct DegridItem {
   int layer, x0, y0;
 };
 
-__device__ __forceinline__ DegridItem degridItem(const GridArgs& a, uint32_t item,
-                                                 uint32_t binLo, uint32_t binHi,
-                                                 const uint32_t* __restrict__ binStart,
-                                                 const uint32_t* __restrict__ itemStart,
-                                                 const uint4* __restrict__ items) {
+__device__ __forceinline__ DegridItem degridItem(const GridArgs& a,
+                                                 const uint4* __restrict__ items, uint32_t i) {
   DegridItem d;
-  d.wi = workItem(items, itemStart[binLo] + item);
+  d.wi = workItem(items, i);
   d.layer = int(d.wi.bin / uint32_t(a.tilesPerLayer));
   const int rem = int(d.wi.bin - uint32_t(d.layer) * uint32_t(a.tilesPerLayer));
   const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
@@ -2133,28 +2128,44 @@ __device__ __forceinline__ float2 subgridCell(const GridArgs& a, const DegridIte
                 cellIndex(gx, gy, a.ga.W, a.ga.blocked)];
 }
 
+// The subgrid of 16 x 16 tiles and K = 7 in the blocked layout: 22 columns by
+// 11 pairs of rows, one pair (16 bytes of a column's 32-byte group) per thread
+// and image, the lanes over whole lines. (A load per cell in row order touched
+// every group four times and spent two divisions by run-time sizes and two
+// remainders on each address.)
+constexpr int kFastSub = 22, kFastPairs = kFastSub * kFastSub / 2;
+
+struct SubgridSlot {
+  int cx, cy;  // column, first row of the pair
+};
+
+__device__ __forceinline__ SubgridSlot subgridSlot(int s) {
+  // five whole row groups (2 pairs x 22 columns each), then the last pair
+  constexpr int kWhole = 5 * 2 * kFastSub;
+  if (s >= kWhole) return SubgridSlot{s - kWhole, 20};
+  const int g = s / (2 * kFastSub), r = s - g * 2 * kFastSub;
+  return SubgridSlot{r >> 1, 4 * g + 2 * (r & 1)};
+}
+
 // The primary records of one item, degridded from its subgrid `sub` in LDS:
-// wave w reads records w * 64 + lane + k * blockDim; qn (wave-uniform)
-// primary records wait in the wave's queue, at most 63 between batches.
+// wave w reads records w * 64 + lane + k * blockDim (the first are loaded by
+// the caller, the next while these are degridded); qn (wave-uniform) primary
+// records wait in the wave's queue, at most 63 between batches.
 template <int NIMG, int KK>
 __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkItem& wi,
-                                                  const uint2* __restrict__ recs,
+                                                  const uint2* __restrict__ recs, uint2 rec,
                                                   const float* kt, const float2* sub,
-                                                  uint2* queue, const double* __restrict__ uvw,
-                                                  const double* __restrict__ wl,
+                                                  uint2* queue, uint32_t byOS,
                                                   float2* __restrict__ out) {
   const int lane = int(threadIdx.x & 63u);
   const unsigned long long below = (1ull << lane) - 1ull;
   const uint32_t start = wi.start, count = wi.count;
   int qn = 0;
   for (uint32_t b = threadIdx.x & ~63u; b < count; b += blockDim.x) {
-    const uint32_t it = b + uint32_t(lane);
-    uint2 rec = make_uint2(0u, 0u);
-    bool primary = false;
-    if (it < count) {
-      rec = recs[start + it];
-      primary = ((rec.x >> 30) & 1u) != 0u;
-    }
+    const bool primary = b + uint32_t(lane) < count && ((rec.x >> 30) & 1u) != 0u;
+    const uint32_t itNext = b + blockDim.x + uint32_t(lane);
+    uint2 recNext = make_uint2(0u, 0u);
+    if (itNext < count) recNext = recs[start + itNext];
     const unsigned long long mask = __ballot(primary);
     if (primary) queue[qn + __popcll(mask & below)] = rec;
     qn += __popcll(mask);
@@ -2167,11 +2178,12 @@ __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkI
       waveSync();
       if (lane < left) queue[lane] = tail;
       qn = left;
-      degridRecord<NIMG, KK>(a, mine, kt, sub, a.sg, uvw, wl, out);
+      degridRecord<NIMG, KK>(a, mine, kt, sub, a.sg, byOS, out);
     }
+    rec = recNext;
   }
   waveSync();
-  if (lane < qn) degridRecord<NIMG, KK>(a, queue[lane], kt, sub, a.sg, uvw, wl, out);
+  if (lane < qn) degridRecord<NIMG, KK>(a, queue[lane], kt, sub, a.sg, byOS, out);
 }
 
 // Degridding of one image kind, one work item per workgroup at a time: the
@@ -2181,14 +2193,13 @@ __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkI
 // compacts the primary records of its share of the item into a queue in
 // LDS and degrids them 64 at a time, one record per lane: no lane idles on
 // the secondary records of split footprints.
-template <int NIMG, int KK>
+// FAST: 16 x 16 tiles, K = 7 and the blocked layout (subgridSlot).
+template <int NIMG, int KK, bool FAST>
 __global__ void __launch_bounds__(kThreads)
-degridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
-                  const uint32_t* __restrict__ itemStart, const uint4* __restrict__ items,
-                  const uint2* __restrict__ recs, const float* __restrict__ ktab,
-                  const __half2* __restrict__ khalf, const double* __restrict__ uvw,
-                  const double* __restrict__ wl, const float2* __restrict__ layers,
-                  float2* __restrict__ out) {
+degridTilesKernel(GridArgs a, const uint32_t* __restrict__ itemStart,
+                  const uint4* __restrict__ items, const uint2* __restrict__ recs,
+                  const float* __restrict__ ktab, const __half2* __restrict__ khalf,
+                  const float2* __restrict__ layers, float2* __restrict__ out) {
   extern __shared__ float smem[];
   const int K = KK ? KK : a.ga.K, OS = a.ga.OS, sg2 = a.sg * a.sg;
   float* kt = smem;
@@ -2198,17 +2209,48 @@ degridTilesKernel(GridArgs a, const uint32_t* __restrict__ binStart,
   loadKernelTable(kt, ktab, khalf, OS * K);
   const uint32_t binLo = uint32_t(a.layerLo) * uint32_t(a.tilesPerLayer);
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
-  const uint32_t nItems = passItems(binLo, binHi, itemStart);
+  const uint32_t nItems = passItems(binLo, binHi, itemStart), base = itemStart[binLo];
+  const uint32_t byOS = kernelRowDivisor(OS);
+  const size_t HW = size_t(a.ga.W) * a.ga.H;
+  const SubgridSlot slot = subgridSlot(int(threadIdx.x));
   for (uint32_t item = blockIdx.x; item < nItems; item += gridDim.x) {
     // every lane decodes the item (uniform loads)
-    const DegridItem d = degridItem(a, item, binLo, binHi, binStart, itemStart, items);
-    if (d.wi.count == 0) continue;  // block-uniform
-    __syncthreads();  // previous item's readers are done with sub and the queues
-    for (int cell = threadIdx.x; cell < sg2; cell += blockDim.x)
+    const DegridItem d = degridItem(a, items, base + item);
+    // the first records are on their way while the subgrid is gathered
+    uint2 rec = make_uint2(0u, 0u);
+    if (threadIdx.x < d.wi.count) rec = recs[d.wi.start + threadIdx.x];
+    float4 pair[FAST ? NIMG : 1];
+    if constexpr (FAST) {
+      if (threadIdx.x < kFastPairs) {
+        int gx = d.x0 + slot.cx, gy = d.y0 + slot.cy;
+        if (gx >= a.ga.W) gx -= a.ga.W;
+        if (gy >= a.ga.H) gy -= a.ga.H;
+        const size_t off = cellIndex(gx, gy, a.ga.W, true);
 #pragma unroll
-      for (int gi = 0; gi < NIMG; ++gi) sub[cell * NIMG + gi] = subgridCell(a, d, cell, gi, layers);
+        for (int gi = 0; gi < NIMG; ++gi)
+          pair[gi] = *reinterpret_cast<const float4*>(
+              layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass + (d.layer - a.passStart)) * HW +
+              off);
+      }
+    }
+    __syncthreads();  // previous item's readers are done with sub and the queues
+    if constexpr (FAST) {
+      if (threadIdx.x < kFastPairs) {
+        float2* cell = sub + size_t(slot.cy * kFastSub + slot.cx) * NIMG;
+#pragma unroll
+        for (int gi = 0; gi < NIMG; ++gi) {
+          cell[gi] = make_float2(pair[gi].x, pair[gi].y);
+          cell[kFastSub * NIMG + gi] = make_float2(pair[gi].z, pair[gi].w);
+        }
+      }
+    } else {
+      for (int cell = threadIdx.x; cell < sg2; cell += blockDim.x)
+#pragma unroll
+        for (int gi = 0; gi < NIMG; ++gi)
+          sub[cell * NIMG + gi] = subgridCell(a, d, cell, gi, layers);
+    }
     __syncthreads();
-    degridItemRecords<NIMG, KK>(a, d.wi, recs, kt, sub, queue, uvw, wl, out);
+    degridItemRecords<NIMG, KK>(a, d.wi, recs, rec, kt, sub, queue, byOS, out);
   }
 }
 
@@ -2881,10 +2923,6 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
   // (both image kinds are counted before either is laid out)
   HWS_TRY(ensureAlloc(g, pl.scanScratch, pl.scanScratchCapacity, 2 * 4 * scanBlocks,
                       "plan scan scratch"));
-  if (!pl.hostCounters)
-    HWS_TRY(checkHip(g, hipHostMalloc(reinterpret_cast<void**>(&pl.hostCounters),
-                                      kPlanCounters * sizeof(unsigned long long)),
-                     "plan counters"));
   if (!pl.counters)
     HWS_TRY(checkHip(g, hipMalloc(&pl.counters, kPlanCounters * sizeof(unsigned long long)),
                      "plan counters"));
@@ -3342,11 +3380,6 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
   Plan& pl = g->plan;
   if (!pl.valid) return setLastError(g, HWS_ERR_BAD_STATE, "no binning plan");
   GridArgs a = gridArgs(g, pass);
-  // as many workgroups as are resident at once (the kernel's registers allow
-  // five waves per SIMD at two images): a static share of items per
-  // workgroup, and no second round of workgroups running at low occupancy
-  // (measured: 8 per CU, 13.2 ms per step at the 4096^2 benchmark; 5, 12.2)
-  const int blocks = persistentBlocks(g, g->degridBlocksPerCu);
   const __half2* khalf = g->cfg.precision == HWS_PRECISION_MIXED ? g->dKernelPair : nullptr;
   const size_t ldsMax = maxLdsBytes(g);
   float2* out = reinterpret_cast<float2*>(dVisOut);
@@ -3365,17 +3398,29 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
       for (int i = 0; i < kMaxImages; ++i)
         a.imgs.idx[i] = (i0 + i < kp.nImg) ? kp.img[i0 + i] : 0;
       const size_t lds = gridLdsBytes(g, n, true);
+      // as many workgroups as are resident at once (51, 71, 91 and 111 registers
+      // for one to four images at K = 7): a static share of items per workgroup,
+      // and no second round of workgroups running at low occupancy. One image:
+      // 2.22 ms with five per CU and 1.71 with eight at 6144^2 x 96 layers (2.85
+      // before the paired gather and the records loaded ahead), 89 us and 81 at
+      // 1024^2 (102); two images at 2048^2 x 32 layers: 338 us with five, 332
+      // with seven, 370 with eight (356).
+      constexpr int kResident[kMaxImages] = {8, 7, 5, 4};
+      const int blocks =
+          persistentBlocks(g, g->degridBlocksPerCu ? g->degridBlocksPerCu : kResident[n - 1]);
       switch (n) {
-#define HWS_DEGRID_GO(N, KK)                                                                  \
-  hipLaunchKernelGGL((degridTilesKernel<N, KK>), dim3(blocks), dim3(kThreads), lds, g->stream,   \
-                     a, kp.binStart, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,  \
-                     pl.uvw, pl.wavelengths, reinterpret_cast<const float2*>(g->dLayers), out)
+#define HWS_DEGRID_GO(N, KK, FAST)                                                            \
+  hipLaunchKernelGGL((degridTilesKernel<N, KK, FAST>), dim3(blocks), dim3(kThreads), lds,       \
+                     g->stream, a, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,     \
+                     reinterpret_cast<const float2*>(g->dLayers), out)
 #define HWS_DEGRID_CASE(N)                                                                \
   case N:                                                                                   \
-    if (g->K == 7)                                                                          \
-      HWS_DEGRID_GO(N, 7);                                                                  \
+    if (g->K == 7 && g->blocked && pl.tileSize == 16)                                       \
+      HWS_DEGRID_GO(N, 7, true);                                                            \
+    else if (g->K == 7)                                                                     \
+      HWS_DEGRID_GO(N, 7, false);                                                           \
     else                                                                                    \
-      HWS_DEGRID_GO(N, 0);                                                                  \
+      HWS_DEGRID_GO(N, 0, false);                                                           \
     break;
         HWS_DEGRID_CASE(1)
         HWS_DEGRID_CASE(2)
