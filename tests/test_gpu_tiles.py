@@ -1,0 +1,101 @@
+"""Gridding and degridding at the edges of tiles, batches and work items,
+against the oracle's restatement of WStackingGridder<float> on the same
+samples. Tolerances as for the other parity tests (relative L2: 1e-5 for the
+reference precision, 3e-5 for the mixed one; the oracle's own float-double
+spread is about 1e-6).
+
+- Sizes that 16 does not divide take 16 x 16 uv tiles with a cut last tile
+  where that holds K - 1 cells (12 at 60, 8 at 56, 72 and 120); 84 and 36 leave 4
+  and keep a tile that divides them.
+- A work item's records are gridded 64 at a time, a bin's in items of
+  work_chunk, with the next batch loaded ahead: counts about both.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+C_LIGHT = 299792458.0
+TOL = {"reference": 1e-5, "mixed": 3e-5}
+
+
+def rel(a, b):
+    a, b = np.asarray(a, np.complex128).ravel(), np.asarray(b, np.complex128).ravel()
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def both_ways(oracle, w, h, dl, uvw, wl, vis, nw, K, precision, chunk=0):
+    """Invert and predict on the device and by the oracle; compared."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    uvw_l = (uvw[:, None, :] / wl[None, :, None]).reshape(-1, 3)
+    maxw = float(np.abs(uvw_l[:, 2]).max())
+    ref = oracle.RefGridder(w, h, dl, dl, 1, K, 63, "float")
+    ref.prepare_w_layers(nw, 1e12, 0.0, maxw)
+    ref.start_inversion_pass(0)
+    ref.add_samples(uvw_l, vis.reshape(-1))
+    ref.finish_inversion_pass()
+    ref.finalize_image(1.0)
+    want = ref.image()
+    model = np.random.default_rng(w + h).standard_normal((h, w)).astype(np.float32)
+    pred = oracle.RefGridder(w, h, dl, dl, 1, K, 63, "float")
+    pred.prepare_w_layers(nw, 1e12, 0.0, maxw)
+    pred.initialize_prediction(model)
+    pred.start_prediction_pass(0)
+    want_v = pred.sample(uvw_l)
+
+    g = wsclean_amd.DeviceGridder(w, h, dl, dl, K, 63, precision=precision, work_chunk=chunk)
+    g.prepare_w_layers(nw, 0.0, maxw)
+    d_vis = torch.from_numpy(vis).to(dev)
+    g.plan(torch.from_numpy(uvw).to(dev), torch.from_numpy(wl).to(dev))
+    img = torch.zeros((1, h, w), dtype=torch.float32, device=dev)
+    g.invert(d_vis, 1.0, img)
+    out = torch.empty_like(d_vis)
+    g.predict(torch.from_numpy(model).to(dev)[None], None, out)
+    g.synchronize()
+    stats = g.stats()
+    g.close()
+    assert rel(img.cpu().numpy()[0], want) < TOL[precision]
+    got = out.cpu().numpy().reshape(-1)
+    ok = np.isfinite(want_v)
+    assert np.array_equal(ok, np.isfinite(got)) and ok.any()
+    assert rel(got[ok], want_v[ok]) < TOL[precision]
+    return stats
+
+
+@pytest.mark.parametrize("precision", ["reference", "mixed"])
+@pytest.mark.parametrize("w,h,K,tiles", [(60, 60, 7, 16), (56, 72, 7, 20), (72, 56, 9, 20),
+                                         (120, 60, 7, 32), (84, 84, 7, 49), (36, 60, 7, 15)])
+def test_cut_tiles_match_oracle(oracle, w, h, K, tiles, precision):
+    rng = np.random.default_rng(w * 7 + h)
+    dl = 0.004
+    wl = C_LIGHT / np.linspace(120e6, 150e6, 4)
+    # the whole uv plane, so that footprints lie across every tile edge and
+    # wrap round both axes
+    umax = 0.499 / dl * wl.min()
+    uvw = np.column_stack([rng.uniform(-umax, umax, 700), rng.uniform(-umax, umax, 700),
+                           rng.uniform(-40, 40, 700)])
+    vis = (rng.standard_normal((700, 4, 1)) + 1j * rng.standard_normal((700, 4, 1))
+           ).astype(np.complex64)
+    s = both_ways(oracle, w, h, dl, uvw, wl, vis, 3, K, precision)
+    assert s["tiles_total"] == 3 * tiles
+    # and with bins split into several items, summed from partial tiles
+    s = both_ways(oracle, w, h, dl, uvw, wl, vis, 1, K, precision, chunk=16)
+    assert s["chunks"] > s["bins_used"]
+
+
+@pytest.mark.parametrize("precision", ["reference", "mixed"])
+@pytest.mark.parametrize("n,chunk", [(1, 0), (63, 0), (64, 0), (65, 0), (129, 64), (257, 64),
+                                     (1024, 0), (1025, 0), (4097, 100)])
+def test_records_about_batches_and_items(oracle, n, chunk, precision):
+    rng = np.random.default_rng(n)
+    w, dl = 64, 0.004
+    wl = C_LIGHT / np.array([140e6])
+    # every sample in one uv cell (one bin, plus its neighbours' halves)
+    uvw = np.column_stack([rng.uniform(-2, 2, n) + 30.0, rng.uniform(-2, 2, n) - 20.0,
+                           rng.uniform(5, 30, n)])
+    vis = (rng.standard_normal((n, 1, 1)) + 1j * rng.standard_normal((n, 1, 1))
+           ).astype(np.complex64)
+    both_ways(oracle, w, w, dl, uvw, wl, vis, 2, 7, precision, chunk)

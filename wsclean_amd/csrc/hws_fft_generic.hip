@@ -161,7 +161,7 @@ hws_status fft2dGeneric(hws_gridder* g, float2* data, int nbatch, int sign,
     rs.layer0 = cs.layer0 = sparse->layer0;
     rs.tilesY = cs.tilesY = sparse->tilesY;
     rs.tshift = cs.tshift = sparse->tshift;
-    rs.tilesX = cs.tilesX = W >> sparse->tshift;
+    rs.tilesX = cs.tilesX = g->plan.tilesX;
     if (sign > 0) {
       rs.bits = sparse->occ;
       cs.bits = sparse->rowLive;

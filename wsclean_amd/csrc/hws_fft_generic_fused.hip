@@ -49,7 +49,7 @@ fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nba
   const int r0 = rblk * L;
   const size_t HW = size_t(W) * H;
   float2* rowBase = data + size_t(r0 >> 2) * 4 * W + (r0 & 3);
-  const int tilesX = W >> tshift;
+  const int tilesX = (W + (1 << tshift) - 1) >> tshift;
   float re[kMaxValues], imv[CPLX ? kMaxValues : 1];
   double np[kMaxValues];
   auto cell = [&](int slot, int x, int f) {
@@ -253,7 +253,7 @@ size_t colsProjectGenericLds(int H, int nLayersInPass, int tilesY) {
 bool colsProjectGenericSupported(const hws_gridder* g, int nLayersInPass, size_t maxLds) {
   const int t = threadsFor(g->colPlan, 1, true);
   return t != 0 && t <= 512 &&
-         colsProjectGenericLds(g->H, nLayersInPass, g->H / g->plan.tileSize) <= maxLds;
+         colsProjectGenericLds(g->H, nLayersInPass, g->plan.tilesY) <= maxLds;
 }
 
 void launchColsProjectGeneric(hws_gridder* g, const ColsProjectArgs& a, bool cplx,

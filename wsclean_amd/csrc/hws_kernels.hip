@@ -210,8 +210,8 @@ struct KindArgs {
 
 // The uv tiles a sample's footprint touches. Footprint cells run from
 // (xs, ys) (centre minus K/2, wrapped into the grid) for K cells per axis;
-// with tileSize >= K - 1 and tiles dividing the grid they touch at most two
-// tiles per axis: tile A holding the first cell and, if different, tile B
+// with tileSize >= K - 1 and tiles dividing the grid (or the last one at least
+// K - 1 wide) they touch at most two tiles per axis: tile A holding the first cell and, if different, tile B
 // holding the last (possibly wrapped round to tile 0). For each tile the
 // footprint start relative to the tile origin is xo in [-(K-1), T).
 struct TileSpan {
@@ -1386,6 +1386,7 @@ gridCellsKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
       const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
       const int x = tx * T + cx, y0 = ty * T + cy0;
+      if (x < a.ga.W && y0 < a.ga.H)  // (as in the matrix-core kernels)
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) {
         float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
@@ -1694,6 +1695,9 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
       const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
       const int x = tx * T + li, y0 = ty * T + 4 * lk;
+      // (cells past the edge of a cut tile belong to no cell of the layer; a
+      // group of four rows is in it or not)
+      if (x < a.ga.W && y0 < a.ga.H)
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) {
         float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
@@ -1980,6 +1984,9 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
       const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
       const int x = tx * T + li, y0 = ty * T + 4 * lg;
+      // (cells past the edge of a cut tile belong to no cell of the layer; a
+      // group of four rows is in it or not)
+      if (x < a.ga.W && y0 < a.ga.H)
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) {
         float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
@@ -2284,12 +2291,12 @@ reducePartialsKernel(GridArgs a, const uint32_t* __restrict__ extraStart,
     if (bin < binLo || bin >= binHi) continue;  // of another pass (workgroup-uniform)
     const uint32_t first = extraStart[bin];
     const int c = int(grp) * kCells + cl;
-    const bool valid = c < T2;
     const uint32_t nEx = extraStart[bin + 1] - first;
     const int layer = int(bin / uint32_t(a.tilesPerLayer));
     const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
     const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
     const int cy = c / T, cx = c - cy * T;
+    const bool valid = c < T2 && tx * T + cx < a.ga.W && ty * T + cy < a.ga.H;
 #pragma unroll
     for (int gi = 0; gi < NIMG; ++gi) {
       // part p of a cell sums the partial tiles p, p + P, p + 2P, ... (P
@@ -2913,8 +2920,9 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
   pl.uvw = dUvw;
   pl.wavelengths = dWl;
   pl.tileSize = g->tileSize;
-  pl.tilesX = g->W / pl.tileSize;
-  pl.tilesY = g->H / pl.tileSize;
+  // (the last tile of an axis may hold less than a whole one, see edgeTiles)
+  pl.tilesX = (g->W + pl.tileSize - 1) / pl.tileSize;
+  pl.tilesY = (g->H + pl.tileSize - 1) / pl.tileSize;
   const size_t tpl = size_t(pl.tilesX) * pl.tilesY;
   pl.nbins = tpl * size_t(g->nW);
   if (pl.nbins >= 0xFFFFFFFFull)
