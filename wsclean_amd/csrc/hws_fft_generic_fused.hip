@@ -4,6 +4,8 @@
 // w-projection.
 #include "hws_fft_generic.h"
 
+#include <algorithm>
+
 namespace hws {
 
 namespace {
@@ -36,11 +38,12 @@ __device__ __forceinline__ void firstStageCells(int n, int tid, int nthr, const 
 // first stage), and then, layer after layer, forms each cell's w-phased
 // input (modelTerm, as modelCell forms it), transforms the rows and writes
 // the tile columns the columns pass reads (colNeed: one bit per (layer, tile
-// column)). grid (H / L).
+// column)). grid (H / L, layer groups): group blockIdx.y takes perGroup
+// consecutive layers.
 template <bool REF, bool CPLX, int L>
 __global__ void __launch_bounds__(1024)
 fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nbatch,
-                                unsigned long long radices, const float2* __restrict__ tw,
+                                int perGroup, unsigned long long radices, const float2* __restrict__ tw,
                                 ModelSource ms, const uint32_t* __restrict__ colNeed,
                                 int tshift) {
   extern __shared__ float2 lds[];
@@ -77,8 +80,9 @@ fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nba
     case 7: firstStageCells<7, L>(W, tid, nthr, cell); break;
     default: break;
   }
+  const int bEnd = min(nbatch, (int(blockIdx.y) + 1) * perGroup);
 #pragma unroll 1
-  for (int b = 0; b < nbatch; ++b) {
+  for (int b = int(blockIdx.y) * perGroup; b < bEnd; ++b) {
     const int layer = ms.layer0 + b;
     const double w = layerToW(ms.map, layer);
     float2* base = rowBase + size_t(b) * HW;
@@ -225,9 +229,18 @@ void launchModelLayersGeneric(int threads, int lines, dim3 grid, size_t lds, hip
                               const float2* tw, const ModelSource& ms, const uint32_t* colNeed,
                               int tshift) {
   const bool cplx = ms.cplx != 0;
+  // At least kModelGroups workgroups, in layer groups of at least two (a group
+  // computes its rows' n' anew): 1500 x 1260 has 315 four-row workgroups, which
+  // left some CUs with two and others with one (24 layers: 420 us an image in
+  // one group, 280 in four).
+  constexpr int kModelGroups = 1024;
+  const int rowBlocks = int(grid.x);
+  const int groups = std::min((nbatch + 1) / 2, (kModelGroups + rowBlocks - 1) / rowBlocks);
+  const int per = (nbatch + groups - 1) / groups;
+  grid.y = unsigned((nbatch + per - 1) / per);
 #define HWS_MODEL_GENERIC(C, LL)                                                                \
   hipLaunchKernelGGL((fftRowsModelLayersGenericKernel<false, C, LL>), grid, dim3(threads), lds,  \
-                     st, data, W, H, nbatch, rad, tw, ms, colNeed, tshift)
+                     st, data, W, H, nbatch, per, rad, tw, ms, colNeed, tshift)
   if (lines == 4) {
     if (cplx) HWS_MODEL_GENERIC(true, 4);
     else HWS_MODEL_GENERIC(false, 4);
