@@ -453,11 +453,13 @@ hws_status hws_create(const hws_config* c, hws_gridder** out) {
     g->tileSize = best ? best : 32;
     // Sizes that 16 does not divide take 16 x 16 tiles all the same where the
     // layers are blocked and a cut last tile is at least K - 1 wide (edgeTiles):
-    // the matrix-core grid kernels and the sparse, fused transforms need the 16
+    // the FP32 matrix-core grid kernel (whose padded table has to fit) and the
+    // sparse, fused transforms need the 16
     // (1500 x 1260, two images, 24 layers, 3.2 M samples: 4.08 ms a step in
     // tiles of 20, 3.28 ms so).
     if (!c->tile_size && best && best != 16 && g->blocked && edgeTiles(g->W, K) &&
-        edgeTiles(g->H, K) && c->precision != HWS_PRECISION_PLAIN_FP32)
+        edgeTiles(g->H, K) && paddedKernelTable(g) &&
+        c->precision != HWS_PRECISION_PLAIN_FP32)
       g->tileSize = 16;
   }
   if ((st = buildF16Table(g)) != HWS_OK) return bail(st);

@@ -618,6 +618,9 @@ __host__ __device__ inline void cellOf(size_t p, int W, bool blocked, int& x, in
 }
 
 bool blockedLayoutSupported(int W, int H);
+// Whether the grid kernels' zero-padded table for 16 x 16 tiles fits their LDS
+// (oversampling up to 221 at K = 7).
+bool paddedKernelTable(const hws_gridder* g);
 // Builds dF16Table where the mixed precision's FP16 grid kernel reads its
 // padded table from device memory (no-op otherwise).
 hws_status buildF16Table(hws_gridder* g);

@@ -2817,10 +2817,14 @@ bool f16TableGlobal(const hws_gridder* g) {
   return !cellTablePadded(g->K, g->OS, 16) && size_t(g->OS) * paddedRow(g->K, 16) < 65536;
 }
 
-// The mixed precision grids on the FP16 matrix cores (split operands).
+// The mixed precision grids on the FP16 matrix cores (split operands). Cut
+// tiles (sizes 16 does not divide) stay with FP32 products, as those sizes had
+// them before they took 16 x 16 tiles: the split adds 1.6e-7 to a layer, which
+// would show (2.7e-7 against 2.3e-7 from the 64-bit evaluation).
 bool mfmaF16(const hws_gridder* g) {
-  return g->plan.tileSize == 16 && !g->noMfma && g->cfg.precision == HWS_PRECISION_MIXED &&
-         !g->noF16Mfma && (cellTablePadded(g->K, g->OS, 16) || f16TableGlobal(g));
+  return g->plan.tileSize == 16 && g->W % 16 == 0 && g->H % 16 == 0 && !g->noMfma &&
+         g->cfg.precision == HWS_PRECISION_MIXED && !g->noF16Mfma &&
+         (cellTablePadded(g->K, g->OS, 16) || f16TableGlobal(g));
 }
 
 size_t gridLdsBytes(const hws_gridder* g, int nimg, bool degrid) {
@@ -2880,6 +2884,8 @@ uint32_t workChunk(const hws_gridder* g, size_t nSamples) {
 }
 
 }  // namespace
+
+bool paddedKernelTable(const hws_gridder* g) { return cellTablePadded(g->K, g->OS, 16); }
 
 hws_status buildF16Table(hws_gridder* g) {
   if (!f16TableGlobal(g) || g->cfg.precision != HWS_PRECISION_MIXED) return HWS_OK;
