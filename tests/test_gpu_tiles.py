@@ -99,3 +99,41 @@ def test_records_about_batches_and_items(oracle, n, chunk, precision):
     vis = (rng.standard_normal((n, 1, 1)) + 1j * rng.standard_normal((n, 1, 1))
            ).astype(np.complex64)
     both_ways(oracle, w, w, dl, uvw, wl, vis, 2, 7, precision, chunk)
+
+
+@pytest.mark.parametrize("w,precision", [(60, "reference"), (60, "mixed"), (64, "reference"),
+                                         (64, "mixed")])
+def test_sums_of_dense_bins_keep_their_precision(oracle, w, precision):
+    """Work items of 8192 records of noise about one uv cell in each of sixteen
+    tiles, against the 64-bit oracle. The batches of 64 are summed on their own
+    and then added, so that a cell's error is that of two short sums: with FP32
+    roundings of at most u = 2^-24 / sqrt(3) rms and the partial sums of noise
+    growing as sqrt(k), n additions leave u sqrt(n / 2), that is 5.7 u within a
+    batch and 8 u over the 128 batches, and the kernel values and products 2 u:
+    10 u = 3.4e-7, and half as much again for the scatter of sixteen sums
+    (measured: 2.2e-7 to 3.1e-7; a running sum of the 2048 matrix products, 32 u
+    and more: 1.5e-6 to 2.2e-6)."""
+    import wsclean_amd
+    rng = np.random.default_rng(w)
+    n, dl = 8192, 0.004
+    wl = C_LIGHT / np.array([140e6])
+    # footprints of 7 cells about these lie inside one tile
+    at = np.repeat(np.array([(x, y) for x in (8, 24, -20, -8) for y in (8, 24, -20, -8)]), n, 0)
+    uvw = np.column_stack([(at + rng.uniform(-0.4, 0.4, at.shape)) * wl[0] / (w * dl),
+                           rng.uniform(1, 2, len(at))])
+    vis = (rng.standard_normal((len(at), 1, 1)) + 1j * rng.standard_normal((len(at), 1, 1))
+           ).astype(np.complex64)
+    uvw_l = (uvw[:, None, :] / wl[None, :, None]).reshape(-1, 3)
+    maxw = float(uvw_l[:, 2].max())
+    ref = oracle.RefGridder(w, w, dl, dl, 1, 7, 63, "double")
+    ref.prepare_w_layers(1, 1e12, 0.0, maxw)
+    ref.start_inversion_pass(0)
+    ref.add_samples(uvw_l, vis.reshape(-1))
+    g = wsclean_amd.WStackingGridder(w, w, dl, dl, 7, 63, precision=precision, work_chunk=n)
+    g.prepare_w_layers(1, 0.0, 0.0, maxw)
+    g.start_inversion_pass(0)
+    g.add_data(uvw, wl, vis)
+    e = rel(g.get_gridded_uv_layer(0, image=0), ref.layer(0))
+    g.close()
+    print(f"{w} {precision}: {e:.2e}")
+    assert e < 15 * 2.0 ** -24 / np.sqrt(3.0)

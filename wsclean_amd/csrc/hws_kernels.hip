@@ -1568,6 +1568,14 @@ __device__ __forceinline__ bool advance(BatchStream<NIMG, ROT>& s,
 // 4 (lane div 16) ..+3). Records are staged in the wave's LDS slice 64 at a
 // time; lane i + 16 k reads record u0 + k of each group of four and looks
 // up its own row (ky) and column (kx) in the zero-padded kernel table.
+// A batch of 64 records is summed on its own and then added to the tile: a
+// running sum over an item's 1024 to 8192 records rounds against the whole sum
+// each time, and left 1.2 to 2.5e-7 on the layers of compact arrays at 300^2 (1.2
+// million samples) where this leaves 0.5 to 1.3e-7 (and the private-tile kernel,
+// which sums runs of records in registers, 1.0 to 2.2e-7). The additions are one
+// in sixteen of the products and cost nothing that could be measured (2048^2 in the
+// reference precision, 6 M samples: 259 and 251 us for one image, 844 and 872 for
+// four, runs differing by 5 %).
 // Work items come from the work queue as in gridCellsKernel.
 constexpr int kMfmaWaves = 4;
 constexpr int kMfmaThreads = 64 * kMfmaWaves;
@@ -1643,6 +1651,9 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       for (int gi = 0; gi < NIMG; ++gi) myVis[lane * NIMG + gi] = v[gi];
       waveSync();
       bs.valNext = loadBatch<NIMG, ROT>(a, vis, bs.recNext, bs.validNext);
+      floatx4 d[2 * NIMG];
+#pragma unroll
+      for (int e = 0; e < 2 * NIMG; ++e) d[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
       // all 64 staged records, sixteen (four groups of four) per round with
       // their LDS reads issued before the first product; the staging is zero
       // past the item's end, and a fully unrolled batch keeps the
@@ -1671,12 +1682,14 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
         for (int q = 0; q < 4; ++q)
 #pragma unroll
           for (int gi = 0; gi < NIMG; ++gi) {
-            acc[2 * gi] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[q][gi].x * ky[q], bx[q],
-                                                               acc[2 * gi], 0, 0, 0);
-            acc[2 * gi + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[q][gi].y * ky[q], bx[q],
-                                                                   acc[2 * gi + 1], 0, 0, 0);
+            d[2 * gi] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[q][gi].x * ky[q], bx[q],
+                                                             d[2 * gi], 0, 0, 0);
+            d[2 * gi + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[q][gi].y * ky[q], bx[q],
+                                                                 d[2 * gi + 1], 0, 0, 0);
           }
       }
+#pragma unroll
+      for (int e = 0; e < 2 * NIMG; ++e) acc[e] += d[e];
       waveSync();  // the staging is rewritten next batch
     }
     if (!bs.last) continue;
@@ -2819,8 +2832,8 @@ bool f16TableGlobal(const hws_gridder* g) {
 
 // The mixed precision grids on the FP16 matrix cores (split operands). Cut
 // tiles (sizes 16 does not divide) stay with FP32 products, as those sizes had
-// them before they took 16 x 16 tiles: the split adds 1.6e-7 to a layer, which
-// would show (2.7e-7 against 2.3e-7 from the 64-bit evaluation).
+// them before they took 16 x 16 tiles: with the split operands 1500 x 1260 was
+// further from the 64-bit evaluation (2.7e-7 against 2.3e-7).
 bool mfmaF16(const hws_gridder* g) {
   return g->plan.tileSize == 16 && g->W % 16 == 0 && g->H % 16 == 0 && !g->noMfma &&
          g->cfg.precision == HWS_PRECISION_MIXED && !g->noF16Mfma &&
