@@ -137,3 +137,72 @@ def test_sums_of_dense_bins_keep_their_precision(oracle, w, precision):
     g.close()
     print(f"{w} {precision}: {e:.2e}")
     assert e < 15 * 2.0 ** -24 / np.sqrt(3.0)
+
+
+@pytest.mark.parametrize("K", [1, 3, 5, 7, 9, 11, 13, 15])
+@pytest.mark.parametrize("w,h", [(120, 60), (64, 96)])
+def test_degridding_of_one_to_four_images(oracle, w, h, K):
+    """The kernel sizes and image counts of the degridding kernel, footprints
+    about every tile edge (60 and 120 leave a cut tile up to K = 9 and K = 13)."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(w + K)
+    dl, nw = 0.003, 2
+    wl = C_LIGHT / np.array([120e6, 150e6])
+    umax = 0.45 / dl * wl.min()
+    uvw = np.column_stack([rng.uniform(-umax, umax, 500), rng.uniform(-umax, umax, 500),
+                           rng.uniform(-30, 30, 500)])
+    uvw_l = (uvw[:, None, :] / wl[None, :, None]).reshape(-1, 3)
+    maxw = float(np.abs(uvw_l[:, 2]).max())
+    model = rng.standard_normal((4, h, w)).astype(np.float32)
+    want = []
+    for m in model:
+        o = oracle.RefGridder(w, h, dl, dl, 1, K, 63, "float")
+        o.prepare_w_layers(nw, 1e12, 0.0, maxw)
+        o.initialize_prediction(m)
+        o.start_prediction_pass(0)
+        want.append(o.sample(uvw_l))
+    d_uvw, d_wl = torch.from_numpy(uvw).to(dev), torch.from_numpy(wl).to(dev)
+    for n in (1, 2, 3, 4):
+        g = wsclean_amd.DeviceGridder(w, h, dl, dl, K, 63, precision="reference", n_images=n)
+        g.prepare_w_layers(nw, 0.0, maxw)
+        g.plan(d_uvw, d_wl)
+        out = torch.empty((500, 2, n), dtype=torch.complex64, device=dev)
+        g.predict(torch.from_numpy(model[:n]).to(dev), None, out)
+        g.synchronize()
+        g.close()
+        got = out.cpu().numpy().reshape(-1, n)
+        for k in range(n):
+            ok = np.isfinite(want[k])
+            assert np.array_equal(ok, np.isfinite(got[:, k])) and ok.any()
+            assert rel(got[ok, k], want[k][ok]) < TOL["reference"], (n, k)
+
+
+def test_degridding_four_images_takes_less_than_four_of_one():
+    """Reading four images' cells must not cost more than four launches of one
+    (with the images interleaved in LDS: 5.4 times one image; in planes: 2.1)."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(3)
+    w, K, nrow, nchan = 1000, 9, 100000, 32
+    dl = 0.0005
+    wl = C_LIGHT / np.linspace(120e6, 168e6, nchan)
+    umax = 0.2 / dl * wl.min()
+    uvw = np.column_stack([rng.uniform(-umax, umax, nrow), rng.uniform(-umax, umax, nrow),
+                           rng.uniform(0, 30, nrow)])
+    d_uvw, d_wl = torch.from_numpy(uvw).to(dev), torch.from_numpy(wl).to(dev)
+    ms = {}
+    for n in (1, 4):
+        g = wsclean_amd.DeviceGridder(w, w, dl, dl, K, 63, n_images=n)
+        g.prepare_w_layers(4, 0.0, float(uvw[:, 2].max() / wl.min()))
+        g.plan(d_uvw, d_wl)
+        model = torch.ones((n, w, w), dtype=torch.float32, device=dev)
+        out = torch.empty((nrow, nchan, n), dtype=torch.complex64, device=dev)
+        times = []
+        for _ in range(9):
+            g.predict(model, None, out)
+            times.append(g.stats()["ms_grid"])
+        g.close()
+        ms[n] = sorted(times)[4]
+    print(f"degridding: {ms}")
+    assert ms[4] < 4 * ms[1]

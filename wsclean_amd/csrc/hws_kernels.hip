@@ -2036,69 +2036,76 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
   } while (advance(bs, items, base, nItems, wq));
 }
 
-// The visibilities of one primary record from the subgrid around its tile
-// (sub: the NIMG images of a cell interleaved, row pitch sg cells). KK: the
-// kernel size when it is fixed at compile time (0: a.ga.K). The taps are
-// summed rows outer, columns inner, as the runtime-K form sums them.
+// The subgrid of NIMG images in LDS, `cells` to a plane: a plane for every two
+// images, whose cells are 16 bytes, then one for the odd image, whose cells are
+// 8. The lanes of a wave read cells far apart (the records of a bin of a 16 x 16
+// tile come in no order of place), so that bank conflicts bound this kernel: a
+// plane's cells take one read each and fall on all banks, where the 8-byte reads
+// of cells interleaved by two images fell on half of them and of four on a
+// quarter. With that and the count of taps known at compile time for every
+// kernel size (the x kernel values stay in registers), 1000^2 x 12 layers, 12 M
+// samples, one to four images:
+//   K = 9: 449, 1006, 924, 2415 us -> 336, 386, 680, 699
+//   K = 7: 208, 234, 535, 536 us -> 207, 236, 391, 418
+template <int NIMG>
+struct Subgrid {
+  float4* pairs;  // [NIMG / 2][cells]
+  float2* last;   // [cells] (odd NIMG)
+  int cells;
+
+  __device__ __forceinline__ Subgrid(float* at, int n)
+      : pairs(reinterpret_cast<float4*>(at)),
+        last(reinterpret_cast<float2*>(at) + size_t(NIMG / 2) * 2 * n),
+        cells(n) {}
+  __device__ __forceinline__ void set(int cell, int gi, float2 v) const {
+    if (NIMG % 2 != 0 && gi == NIMG - 1)
+      last[cell] = v;
+    else
+      reinterpret_cast<float2*>(pairs + (gi / 2) * cells + cell)[gi & 1] = v;
+  }
+};
+
+// The visibilities of one primary record from the subgrid (rows of sg cells)
+// around its tile, KK taps an axis, rows outer, columns inner.
 template <int NIMG, int KK>
 __device__ __forceinline__ void degridRecord(const GridArgs& a, uint2 rec,
                                              const float* __restrict__ kt,
-                                             const float2* __restrict__ sub, int sg,
-                                             uint32_t byOS, float2* __restrict__ out) {
-  const int K = KK ? KK : a.ga.K, OS = a.ga.OS;
+                                             const Subgrid<NIMG>& sub, int sg, uint32_t byOS,
+                                             float2* __restrict__ out) {
+  const int OS = a.ga.OS;
   const uint32_t idx = rec.x & 0x3FFFFFFFu;
   const bool conj = (rec.x >> 31) != 0;
-  const int xo = int(rec.y & 63u) - (K - 1), yo = int((rec.y >> 6) & 63u) - (K - 1);
+  const int xo = int(rec.y & 63u) - (KK - 1), yo = int((rec.y >> 6) & 63u) - (KK - 1);
   const int kk = int(rec.y >> 12);
   const int ky = kernelRow(kk, byOS), kx = kk - ky * OS;
   float2 acc[NIMG];
 #pragma unroll
   for (int gi = 0; gi < NIMG; ++gi) acc[gi] = make_float2(0.0f, 0.0f);
-  if constexpr (KK > 0) {
-    float xk[KK];
+  float xk[KK];
 #pragma unroll
-    for (int i = 0; i < KK; ++i) xk[i] = kt[kx * KK + i];
-    // one row of taps in flight at a time: unrolling the rows hoists every
-    // LDS read of the footprint and leaves one wave per SIMD
+  for (int i = 0; i < KK; ++i) xk[i] = kt[kx * KK + i];
+  // one row of taps in flight at a time: unrolling the rows hoists every
+  // LDS read of the footprint and leaves one wave per SIMD
 #pragma nounroll
-    for (int j = 0; j < KK; ++j) {
-      const float yk = kt[ky * KK + j];
-      const float2* row = sub + size_t((yo + j) * sg + xo) * NIMG;
+  for (int j = 0; j < KK; ++j) {
+    const float yk = kt[ky * KK + j];
+    const int row = (yo + j) * sg + xo;
 #pragma unroll
-      for (int i = 0; i < KK; ++i) {
-        // xKernel[i] * yKernelValue (gridding/wstackinggridder.cpp:668)
-        const float kv = xk[i] * yk;
-        if constexpr (NIMG % 2 == 0) {
+    for (int i = 0; i < KK; ++i) {
+      // xKernel[i] * yKernelValue (gridding/wstackinggridder.cpp:668)
+      const float kv = xk[i] * yk;
 #pragma unroll
-          for (int gp = 0; gp < NIMG / 2; ++gp) {
-            const float4 gv = reinterpret_cast<const float4*>(row + i * NIMG)[gp];
-            acc[2 * gp].x += gv.x * kv;
-            acc[2 * gp].y += gv.y * kv;
-            acc[2 * gp + 1].x += gv.z * kv;
-            acc[2 * gp + 1].y += gv.w * kv;
-          }
-        } else {
-#pragma unroll
-          for (int gi = 0; gi < NIMG; ++gi) {
-            const float2 gv = row[i * NIMG + gi];
-            acc[gi].x += gv.x * kv;
-            acc[gi].y += gv.y * kv;
-          }
-        }
+      for (int gp = 0; gp < NIMG / 2; ++gp) {
+        const float4 gv = sub.pairs[gp * sub.cells + row + i];
+        acc[2 * gp].x += gv.x * kv;
+        acc[2 * gp].y += gv.y * kv;
+        acc[2 * gp + 1].x += gv.z * kv;
+        acc[2 * gp + 1].y += gv.w * kv;
       }
-    }
-  } else {
-    for (int j = 0; j < K; ++j) {
-      const float yk = kt[ky * K + j];
-      const float2* row = sub + size_t((yo + j) * sg + xo) * NIMG;
-      for (int i = 0; i < K; ++i) {
-        const float kv = kt[kx * K + i] * yk;
-#pragma unroll
-        for (int gi = 0; gi < NIMG; ++gi) {
-          const float2 gv = row[i * NIMG + gi];
-          acc[gi].x += gv.x * kv;
-          acc[gi].y += gv.y * kv;
-        }
+      if constexpr (NIMG % 2 != 0) {
+        const float2 gv = sub.last[row + i];
+        acc[NIMG - 1].x += gv.x * kv;
+        acc[NIMG - 1].y += gv.y * kv;
       }
     }
   }
@@ -2174,7 +2181,7 @@ __device__ __forceinline__ SubgridSlot subgridSlot(int s) {
 template <int NIMG, int KK>
 __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkItem& wi,
                                                   const uint2* __restrict__ recs, uint2 rec,
-                                                  const float* kt, const float2* sub,
+                                                  const float* kt, const Subgrid<NIMG>& sub,
                                                   uint2* queue, uint32_t byOS,
                                                   float2* __restrict__ out) {
   const int lane = int(threadIdx.x & 63u);
@@ -2221,12 +2228,13 @@ degridTilesKernel(GridArgs a, const uint32_t* __restrict__ itemStart,
                   const float* __restrict__ ktab, const __half2* __restrict__ khalf,
                   const float2* __restrict__ layers, float2* __restrict__ out) {
   extern __shared__ float smem[];
-  const int K = KK ? KK : a.ga.K, OS = a.ga.OS, sg2 = a.sg * a.sg;
+  const int OS = a.ga.OS, sg2 = a.sg * a.sg;
   float* kt = smem;
-  float2* sub = reinterpret_cast<float2*>(smem + ((OS * K + 3) & ~3));  // [sg2][NIMG]
-  uint2* queue = reinterpret_cast<uint2*>(sub + size_t(NIMG) * sg2) +
+  float* subAt = smem + ((OS * KK + 3) & ~3);
+  const Subgrid<NIMG> sub(subAt, sg2);
+  uint2* queue = reinterpret_cast<uint2*>(subAt + size_t(NIMG) * 2 * sg2) +
                  (threadIdx.x >> 6) * kDegridQueue;
-  loadKernelTable(kt, ktab, khalf, OS * K);
+  loadKernelTable(kt, ktab, khalf, OS * KK);
   const uint32_t binLo = uint32_t(a.layerLo) * uint32_t(a.tilesPerLayer);
   const uint32_t binHi = uint32_t(a.layerHi) * uint32_t(a.tilesPerLayer);
   const uint32_t nItems = passItems(binLo, binHi, itemStart), base = itemStart[binLo];
@@ -2256,18 +2264,18 @@ degridTilesKernel(GridArgs a, const uint32_t* __restrict__ itemStart,
     __syncthreads();  // previous item's readers are done with sub and the queues
     if constexpr (FAST) {
       if (threadIdx.x < kFastPairs) {
-        float2* cell = sub + size_t(slot.cy * kFastSub + slot.cx) * NIMG;
+        const int cell = slot.cy * kFastSub + slot.cx;
 #pragma unroll
         for (int gi = 0; gi < NIMG; ++gi) {
-          cell[gi] = make_float2(pair[gi].x, pair[gi].y);
-          cell[kFastSub * NIMG + gi] = make_float2(pair[gi].z, pair[gi].w);
+          sub.set(cell, gi, make_float2(pair[gi].x, pair[gi].y));
+          sub.set(cell + kFastSub, gi, make_float2(pair[gi].z, pair[gi].w));
         }
       }
     } else {
       for (int cell = threadIdx.x; cell < sg2; cell += blockDim.x)
 #pragma unroll
         for (int gi = 0; gi < NIMG; ++gi)
-          sub[cell * NIMG + gi] = subgridCell(a, d, cell, gi, layers);
+          sub.set(cell, gi, subgridCell(a, d, cell, gi, layers));
     }
     __syncthreads();
     degridItemRecords<NIMG, KK>(a, d.wi, recs, rec, kt, sub, queue, byOS, out);
@@ -3403,6 +3411,25 @@ hws_status markSkipped(hws_gridder* g, float* dVisOut) {
   return HWS_OK;
 }
 
+namespace {
+using DegridKernel = void (*)(GridArgs, const uint32_t*, const uint4*, const uint2*, const float*,
+                              const __half2*, const float2*, float2*);
+
+template <int NIMG>
+DegridKernel degridKernelOf(int K, bool fast) {
+  switch (K) {
+    case 1: return degridTilesKernel<NIMG, 1, false>;
+    case 3: return degridTilesKernel<NIMG, 3, false>;
+    case 5: return degridTilesKernel<NIMG, 5, false>;
+    case 7: return fast ? degridTilesKernel<NIMG, 7, true> : degridTilesKernel<NIMG, 7, false>;
+    case 9: return degridTilesKernel<NIMG, 9, false>;
+    case 11: return degridTilesKernel<NIMG, 11, false>;
+    case 13: return degridTilesKernel<NIMG, 13, false>;
+    default: return degridTilesKernel<NIMG, 15, false>;
+  }
+}
+}  // namespace
+
 hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
   Plan& pl = g->plan;
   if (!pl.valid) return setLastError(g, HWS_ERR_BAD_STATE, "no binning plan");
@@ -3425,7 +3452,12 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
       for (int i = 0; i < kMaxImages; ++i)
         a.imgs.idx[i] = (i0 + i < kp.nImg) ? kp.img[i0 + i] : 0;
       const size_t lds = gridLdsBytes(g, n, true);
-      // as many workgroups as are resident at once (51, 71, 91 and 111 registers
+      const bool fast = g->K == 7 && g->blocked && pl.tileSize == 16;
+      const DegridKernel kernel = n == 1   ? degridKernelOf<1>(g->K, fast)
+                                  : n == 2 ? degridKernelOf<2>(g->K, fast)
+                                  : n == 3 ? degridKernelOf<3>(g->K, fast)
+                                           : degridKernelOf<4>(g->K, fast);
+      // as many workgroups as are resident at once (51, 71, 96 and 115 registers
       // for one to four images at K = 7): a static share of items per workgroup,
       // and no second round of workgroups running at low occupancy. One image:
       // 2.22 ms with five per CU and 1.71 with eight at 6144^2 x 96 layers (2.85
@@ -3435,27 +3467,9 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
       constexpr int kResident[kMaxImages] = {8, 7, 5, 4};
       const int blocks =
           persistentBlocks(g, g->degridBlocksPerCu ? g->degridBlocksPerCu : kResident[n - 1]);
-      switch (n) {
-#define HWS_DEGRID_GO(N, KK, FAST)                                                            \
-  hipLaunchKernelGGL((degridTilesKernel<N, KK, FAST>), dim3(blocks), dim3(kThreads), lds,       \
-                     g->stream, a, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,     \
-                     reinterpret_cast<const float2*>(g->dLayers), out)
-#define HWS_DEGRID_CASE(N)                                                                \
-  case N:                                                                                   \
-    if (g->K == 7 && g->blocked && pl.tileSize == 16)                                       \
-      HWS_DEGRID_GO(N, 7, true);                                                            \
-    else if (g->K == 7)                                                                     \
-      HWS_DEGRID_GO(N, 7, false);                                                           \
-    else                                                                                    \
-      HWS_DEGRID_GO(N, 0, false);                                                           \
-    break;
-        HWS_DEGRID_CASE(1)
-        HWS_DEGRID_CASE(2)
-        HWS_DEGRID_CASE(3)
-        HWS_DEGRID_CASE(4)
-#undef HWS_DEGRID_CASE
-#undef HWS_DEGRID_GO
-      }
+      hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), lds, g->stream,
+                         a, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,
+                         reinterpret_cast<const float2*>(g->dLayers), out);
       HWS_TRY(checkHip(g, hipGetLastError(), "degrid launch"));
     }
   }
