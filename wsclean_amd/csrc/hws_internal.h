@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/hip_wstacking.h"
+#include "hws_rules.h"
 
 namespace hws {
 
@@ -433,8 +434,9 @@ struct hws_gridder {
   // the mixed precision grids with the FP32 matrix-core kernel
   // (HWS_NO_F16_MFMA=1)
   bool noF16Mfma = false;
-  // degridding workgroups per CU (HWS_DEGRID_BLOCKS_PER_CU; 0: by images)
+  // degridding workgroups per CU (HWS_DEGRID_BLOCKS_PER_CU; 0: wholeRounds)
   int degridBlocksPerCu = 0;
+  int degridPerCu[hws::kMaxImages] = {};  // those of a launch of 1, 2, ... images, once known
   // lines (rows or columns) per workgroup of the blocked runtime-radix
   // transforms (HWS_FFT_LINES = 1, 2 or 4; 0: chosen by size)
   int fftLines = 0;

@@ -3428,6 +3428,17 @@ DegridKernel degridKernelOf(int K, bool fast) {
     default: return degridTilesKernel<NIMG, 15, false>;
   }
 }
+
+// Workgroups per CU of a degridding launch (each takes a static share of the
+// items).
+hws_status degridWorkgroupsPerCu(hws_gridder* g, DegridKernel kernel, size_t lds, int& perCu) {
+  int resident = 0;
+  HWS_TRY(checkHip(g, hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                          &resident, reinterpret_cast<const void*>(kernel), kThreads, lds),
+                   "degrid occupancy"));
+  perCu = g->degridBlocksPerCu ? g->degridBlocksPerCu : wholeRounds(resident);
+  return HWS_OK;
+}
 }  // namespace
 
 hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
@@ -3457,17 +3468,9 @@ hws_status degridBinned(hws_gridder* g, float* dVisOut, int pass) {
                                   : n == 2 ? degridKernelOf<2>(g->K, fast)
                                   : n == 3 ? degridKernelOf<3>(g->K, fast)
                                            : degridKernelOf<4>(g->K, fast);
-      // as many workgroups as are resident at once (51, 71, 96 and 115 registers
-      // for one to four images at K = 7): a static share of items per workgroup,
-      // and no second round of workgroups running at low occupancy. One image:
-      // 2.22 ms with five per CU and 1.71 with eight at 6144^2 x 96 layers (2.85
-      // before the paired gather and the records loaded ahead), 89 us and 81 at
-      // 1024^2 (102); two images at 2048^2 x 32 layers: 338 us with five, 332
-      // with seven, 370 with eight (356).
-      constexpr int kResident[kMaxImages] = {8, 7, 5, 4};
-      const int blocks =
-          persistentBlocks(g, g->degridBlocksPerCu ? g->degridBlocksPerCu : kResident[n - 1]);
-      hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), lds, g->stream,
+      int& perCu = g->degridPerCu[n - 1];
+      if (perCu == 0) HWS_TRY(degridWorkgroupsPerCu(g, kernel, lds, perCu));
+      hipLaunchKernelGGL(kernel, dim3(persistentBlocks(g, perCu)), dim3(kThreads), lds, g->stream,
                          a, kp.itemStart, kp.items, kp.recSorted, g->dKernel, khalf,
                          reinterpret_cast<const float2*>(g->dLayers), out);
       HWS_TRY(checkHip(g, hipGetLastError(), "degrid launch"));
