@@ -108,3 +108,49 @@ def test_fused_projection_equals_separate_kernels(w, h, precision, nw, passes):
     assert dv < 1e-6
     assert d < 1e-6
     assert np.abs(im_f[1:3] - im_s[1:3]).max() / np.abs(im_s[1:3]).max() < 1e-6
+
+
+@pytest.mark.parametrize("w,h,precision,nw,passes", [
+    (1680, 1600, "mixed", 5, 1), (1600, 1620, "mixed", 6, 2),
+    # a last uv tile of 8 cells on either axis
+    (1800, 1960, "mixed", 7, 3), (1960, 1800, "reference", 4, 2), (1800, 300, "mixed", 5, 1),
+    (300, 1800, "mixed", 5, 2)])
+def test_fused_runtime_radix_equals_separate_kernels(w, h, precision, nw, passes):
+    """The sizes from which the runtime-radix transforms run fused on one axis
+    or both, with whole and cut uv tiles, as above."""
+    test_fused_projection_equals_separate_kernels(w, h, precision, nw, passes)
+
+
+@pytest.mark.parametrize("w", [300, 600])
+def test_many_layers_of_a_small_image_are_not_transformed_one_after_the_other(w):
+    """48 layers of a small image at a runtime-radix size: invert takes about
+    what the separate transforms take (one workgroup per column, layer after
+    layer, took 2.6 times that at either size)."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    uvw, wl, vis, dl, maxw = _case(w, 2000, seed=w, nimg=1)
+    d_uvw, d_wl = torch.from_numpy(uvw).to(dev), torch.from_numpy(wl).to(dev)
+    d_vis = torch.from_numpy(vis).to(dev)
+    ms = {}
+    for off in ("0", "1"):
+        old = os.environ.get("HWS_NO_FUSED_PROJECT")
+        os.environ["HWS_NO_FUSED_PROJECT"] = off
+        try:
+            g = wsclean_amd.DeviceGridder(w, w, dl, dl, 7, 63, precision="mixed")
+        finally:
+            if old is None:
+                del os.environ["HWS_NO_FUSED_PROJECT"]
+            else:
+                os.environ["HWS_NO_FUSED_PROJECT"] = old
+        g.prepare_w_layers(48, 0.0, maxw)
+        g.plan(d_uvw, d_wl)
+        re = torch.zeros((1, w, w), dtype=torch.float32, device=dev)
+        times = []
+        for _ in range(9):
+            g.invert(d_vis, 1.0, re)
+            s = g.stats()
+            times.append(s["ms_fft"] + s["ms_project"])
+        g.close()
+        ms[off] = sorted(times)[4]
+    print(f"{w}: {ms}")
+    assert ms["0"] < 1.5 * ms["1"]

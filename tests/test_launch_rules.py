@@ -30,3 +30,8 @@ def test_degridding_launches_whole_rounds_of_resident_workgroups(rule):
     residents = list(range(0, 17))
     for r, per in zip(residents, rule([f"wholeRounds({r})" for r in residents])):
         assert per % max(r, 1) == 0 and per >= 5 and per - max(r, 1) < 5
+
+
+def test_runtime_radix_transforms_run_fused_at_long_lines_only(rule):
+    sizes = [60, 300, 600, 840, 1260, 1500, 1600, 1680, 1920, 3072, 6144]
+    assert rule([f"fusedRuntimeRadix({n})" for n in sizes]) == [int(n >= 1600) for n in sizes]

@@ -185,7 +185,8 @@ hws_status fft2dGeneric(hws_gridder* g, float2* data, int nbatch, int sign,
   } else {
     // (the mixed precision: the reference precision's FP64 sincos leaves no
     // registers for the cells it keeps)
-    if (model && sparse && sparse->colNeed && model->precision != HWS_PRECISION_REFERENCE)
+    if (model && sparse && sparse->colNeed && fusedRuntimeRadix(W) &&
+        model->precision != HWS_PRECISION_REFERENCE)
       launchModelLayersGeneric(tr, rl, dim3(H >> rbShift), ldsR, st, data, W, H, nbatch, radR,
                                twRow, msrc, sparse->colNeed, sparse->tshift);
     else if (model && model->precision == HWS_PRECISION_REFERENCE)

@@ -265,7 +265,7 @@ size_t colsProjectGenericLds(int H, int nLayersInPass, int tilesY) {
 
 bool colsProjectGenericSupported(const hws_gridder* g, int nLayersInPass, size_t maxLds) {
   const int t = threadsFor(g->colPlan, 1, true);
-  return t != 0 && t <= 512 &&
+  return fusedRuntimeRadix(g->H) && t != 0 && t <= 512 &&
          colsProjectGenericLds(g->H, nLayersInPass, g->plan.tilesY) <= maxLds;
 }
 
