@@ -1386,36 +1386,37 @@ gridCellsKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
       const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
       const int x = tx * T + cx, y0 = ty * T + cy0;
-      if (x < a.ga.W && y0 < a.ga.H)  // (as in the matrix-core kernels)
+      if (x < a.ga.W && y0 < a.ga.H) {  // (as in the matrix-core kernels)
 #pragma unroll
-      for (int gi = 0; gi < NIMG; ++gi) {
-        float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
-                                 size_t(layer - a.passStart)) * HW;
-        if (R == 4 && a.ga.blocked) {
-          // rows y0 .. y0 + 3 of one column are 32 contiguous bytes
-          float4* dst = reinterpret_cast<float4*>(base + cellIndex(x, y0, a.ga.W, 1));
-          float4 lo = make_float4(acc[0][2 * gi], acc[0][2 * gi + 1], acc[1 % R][2 * gi],
-                                  acc[1 % R][2 * gi + 1]);
-          float4 hi = make_float4(acc[2 % R][2 * gi], acc[2 % R][2 * gi + 1],
-                                  acc[3 % R][2 * gi], acc[3 % R][2 * gi + 1]);
-          if (ACCUM) {
-            const float4 o0 = dst[0], o1 = dst[1];
-            lo.x += o0.x; lo.y += o0.y; lo.z += o0.z; lo.w += o0.w;
-            hi.x += o1.x; hi.y += o1.y; hi.z += o1.z; hi.w += o1.w;
-          }
-          dst[0] = lo;
-          dst[1] = hi;
-        } else {
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            float2* dst = base + cellIndex(x, y0 + r, a.ga.W, a.ga.blocked);
-            float2 val = make_float2(acc[r][2 * gi], acc[r][2 * gi + 1]);
+        for (int gi = 0; gi < NIMG; ++gi) {
+          float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
+                                   size_t(layer - a.passStart)) * HW;
+          if (R == 4 && a.ga.blocked) {
+            // rows y0 .. y0 + 3 of one column are 32 contiguous bytes
+            float4* dst = reinterpret_cast<float4*>(base + cellIndex(x, y0, a.ga.W, 1));
+            float4 lo = make_float4(acc[0][2 * gi], acc[0][2 * gi + 1], acc[1 % R][2 * gi],
+                                    acc[1 % R][2 * gi + 1]);
+            float4 hi = make_float4(acc[2 % R][2 * gi], acc[2 % R][2 * gi + 1],
+                                    acc[3 % R][2 * gi], acc[3 % R][2 * gi + 1]);
             if (ACCUM) {
-              const float2 o = *dst;
-              val.x += o.x;
-              val.y += o.y;
+              const float4 o0 = dst[0], o1 = dst[1];
+              lo.x += o0.x; lo.y += o0.y; lo.z += o0.z; lo.w += o0.w;
+              hi.x += o1.x; hi.y += o1.y; hi.z += o1.z; hi.w += o1.w;
             }
-            *dst = val;
+            dst[0] = lo;
+            dst[1] = hi;
+          } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              float2* dst = base + cellIndex(x, y0 + r, a.ga.W, a.ga.blocked);
+              float2 val = make_float2(acc[r][2 * gi], acc[r][2 * gi + 1]);
+              if (ACCUM) {
+                const float2 o = *dst;
+                val.x += o.x;
+                val.y += o.y;
+              }
+              *dst = val;
+            }
           }
         }
       }
@@ -1710,35 +1711,36 @@ gridMfmaKernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int x = tx * T + li, y0 = ty * T + 4 * lk;
       // (cells past the edge of a cut tile belong to no cell of the layer; a
       // group of four rows is in it or not)
-      if (x < a.ga.W && y0 < a.ga.H)
+      if (x < a.ga.W && y0 < a.ga.H) {
 #pragma unroll
-      for (int gi = 0; gi < NIMG; ++gi) {
-        float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
-                                 size_t(layer - a.passStart)) * HW;
-        const floatx4 re = acc[2 * gi], im = acc[2 * gi + 1];
-        if (a.ga.blocked) {
-          // rows y0 .. y0 + 3 of one column are 32 contiguous bytes
-          float4* dst = reinterpret_cast<float4*>(base + cellIndex(x, y0, a.ga.W, 1));
-          float4 lo = make_float4(re[0], im[0], re[1], im[1]);
-          float4 hi = make_float4(re[2], im[2], re[3], im[3]);
-          if (ACCUM) {
-            const float4 o0 = dst[0], o1 = dst[1];
-            lo.x += o0.x; lo.y += o0.y; lo.z += o0.z; lo.w += o0.w;
-            hi.x += o1.x; hi.y += o1.y; hi.z += o1.z; hi.w += o1.w;
-          }
-          dst[0] = lo;
-          dst[1] = hi;
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float2* dst = base + cellIndex(x, y0 + r, a.ga.W, 0);
-            float2 val = make_float2(re[r], im[r]);
+        for (int gi = 0; gi < NIMG; ++gi) {
+          float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
+                                   size_t(layer - a.passStart)) * HW;
+          const floatx4 re = acc[2 * gi], im = acc[2 * gi + 1];
+          if (a.ga.blocked) {
+            // rows y0 .. y0 + 3 of one column are 32 contiguous bytes
+            float4* dst = reinterpret_cast<float4*>(base + cellIndex(x, y0, a.ga.W, 1));
+            float4 lo = make_float4(re[0], im[0], re[1], im[1]);
+            float4 hi = make_float4(re[2], im[2], re[3], im[3]);
             if (ACCUM) {
-              const float2 o = *dst;
-              val.x += o.x;
-              val.y += o.y;
+              const float4 o0 = dst[0], o1 = dst[1];
+              lo.x += o0.x; lo.y += o0.y; lo.z += o0.z; lo.w += o0.w;
+              hi.x += o1.x; hi.y += o1.y; hi.z += o1.z; hi.w += o1.w;
             }
-            *dst = val;
+            dst[0] = lo;
+            dst[1] = hi;
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float2* dst = base + cellIndex(x, y0 + r, a.ga.W, 0);
+              float2 val = make_float2(re[r], im[r]);
+              if (ACCUM) {
+                const float2 o = *dst;
+                val.x += o.x;
+                val.y += o.y;
+              }
+              *dst = val;
+            }
           }
         }
       }
@@ -1831,6 +1833,7 @@ __device__ __forceinline__ uint32_t lowParts(float x0, float x1, uint32_t h) {
 // Operand layout: lane i + 16 g supplies A[i][8 g + t] and B[8 g + t][i] in
 // its eight halves t (the same k order on both sides, so records may take
 // any k); D as for gridMfmaKernel. Staging, work queue and output as there.
+// Whole tiles only (mfmaF16).
 // GT: the padded table is read from device memory (gkt, gkp: f16TableKernel's
 // output) rather than built in LDS, for oversampling factors whose table does
 // not fit the LDS (above 221 at K = 7); the values are the same.
@@ -1997,9 +2000,6 @@ gridMfmaF16Kernel(GridArgs a, const uint32_t* __restrict__ binStart,
       const int rem = int(bin - uint32_t(layer) * uint32_t(a.tilesPerLayer));
       const int ty = rem / a.ga.tilesX, tx = rem - ty * a.ga.tilesX;
       const int x = tx * T + li, y0 = ty * T + 4 * lg;
-      // (cells past the edge of a cut tile belong to no cell of the layer; a
-      // group of four rows is in it or not)
-      if (x < a.ga.W && y0 < a.ga.H)
 #pragma unroll
       for (int gi = 0; gi < NIMG; ++gi) {
         float2* base = layers + (size_t(a.imgs.idx[gi]) * a.nLayersPass +
