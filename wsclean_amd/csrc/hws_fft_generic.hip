@@ -183,8 +183,8 @@ hws_status fft2dGeneric(hws_gridder* g, float2* data, int nbatch, int sign,
       launchColsGeneric<+1, 0>(tc, cl, gc, ldsC, st, data, W, H, nColBlocks, radC, twCol, cs);
     }
   } else {
-    // (the mixed precision: the reference precision's FP64 sincos leaves no
-    // registers for the cells it keeps)
+    // (the mixed precision: the reference precision's terms leave no registers
+    // for the cells it keeps)
     if (model && sparse && sparse->colNeed && fusedRuntimeRadix(W) &&
         model->precision != HWS_PRECISION_REFERENCE)
       launchModelLayersGeneric(tr, rl, dim3(H >> rbShift), ldsR, st, data, W, H, nbatch, radR,

@@ -39,8 +39,10 @@ __device__ __forceinline__ void firstStageCells(int n, int tid, int nthr, const 
 // input (modelTerm, as modelCell forms it), transforms the rows and writes
 // the tile columns the columns pass reads (colNeed: one bit per (layer, tile
 // column)). grid (H / L, layer groups): group blockIdx.y takes perGroup
-// consecutive layers.
-template <bool REF, bool CPLX, int L>
+// consecutive layers. Mixed precision only: the 1024 threads of the long rows
+// leave 128 registers, and with the reference precision's FP64 sine and cosine
+// 106 to 240 values spill inside the layer loop.
+template <bool CPLX, int L>
 __global__ void __launch_bounds__(1024)
 fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nbatch,
                                 int perGroup, unsigned long long radices, const float2* __restrict__ tw,
@@ -63,9 +65,7 @@ fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nba
     if (xDest >= W) xDest -= W;
     const double m = pixelM(yDest, H, ms.dm, ms.mShift);
     const double l = pixelL(xDest, W, ms.dl, ms.lShift);
-    double v = nPrimeSeries(l, m);
-    if (REF) v = double(float(v));
-    np[slot] = v;
+    np[slot] = nPrimeSeries(l, m);
     const size_t src = size_t(yDest) * W + xDest;
     re[slot] = ms.re[src];
     if (CPLX) imv[slot] = -ms.im[src];
@@ -88,7 +88,7 @@ fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nba
     float2* base = rowBase + size_t(b) * HW;
     const size_t cbit = size_t(layer) * tilesX;
     auto load = [&](int slot, int, int) -> float2 {
-      return modelTerm<REF>(re[slot], CPLX ? imv[slot] : 0.0f, CPLX, w, np[slot]);
+      return modelTerm<false>(re[slot], CPLX ? imv[slot] : 0.0f, CPLX, w, np[slot]);
     };
     auto store = [&](int, int x, int f, float2 v) {
       const size_t bit = cbit + size_t(x >> tshift);
@@ -239,7 +239,7 @@ void launchModelLayersGeneric(int threads, int lines, dim3 grid, size_t lds, hip
   const int per = (nbatch + groups - 1) / groups;
   grid.y = unsigned((nbatch + per - 1) / per);
 #define HWS_MODEL_GENERIC(C, LL)                                                                \
-  hipLaunchKernelGGL((fftRowsModelLayersGenericKernel<false, C, LL>), grid, dim3(threads), lds,  \
+  hipLaunchKernelGGL((fftRowsModelLayersGenericKernel<C, LL>), grid, dim3(threads), lds,  \
                      st, data, W, H, nbatch, per, rad, tw, ms, colNeed, tshift)
   if (lines == 4) {
     if (cplx) HWS_MODEL_GENERIC(true, 4);
