@@ -206,3 +206,99 @@ def test_degridding_four_images_takes_less_than_four_of_one():
         ms[n] = sorted(times)[4]
     print(f"degridding: {ms}")
     assert ms[4] < 4 * ms[1]
+
+
+@pytest.mark.parametrize("precision", ["reference", "mixed"])
+@pytest.mark.parametrize("no_mfma", ["0", "1"])
+def test_cut_tiles_with_images_rotation_batches_and_passes(oracle, monkeypatch, precision,
+                                                           no_mfma):
+    """A last tile of 8 by 12 cells with two real images and a complex one, a
+    shifted and rotated phase centre and bins split into work items: two batches
+    through the host protocol (the second adds to the tiles), then one pass and
+    two on the device, by the matrix-core kernel and (HWS_NO_MFMA=1) the cell
+    kernel."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    monkeypatch.setenv("HWS_NO_MFMA", no_mfma)
+    w, h, dl, nw, n = 120, 60, 0.003, 5, 700
+    shift = (0.006, -0.004)
+    rng = np.random.default_rng(120)
+    wl = C_LIGHT / np.linspace(120e6, 150e6, 3)
+    umax = 0.499 / dl * wl.min()
+    uvw = np.column_stack([rng.uniform(-umax, umax, n), rng.uniform(-umax, umax, n),
+                           rng.uniform(-40, 40, n)])
+    # half of them about the edge of the cut tiles
+    edge = wl.min() / dl * np.array([-9.0 / w, -13.0 / h])
+    uvw[::2, :2] = edge + rng.uniform(-4, 4, (n // 2, 2)) * wl.min() / (dl * np.array([w, h]))
+    vis = (rng.standard_normal((n, 3, 3)) + 1j * rng.standard_normal((n, 3, 3))
+           ).astype(np.complex64)
+    uvw_l = (uvw[:, None, :] / wl[None, :, None]).reshape(-1, 3)
+    maxw = float(np.abs(uvw_l[:, 2]).max())
+    ph = np.exp(-2j * np.pi * (uvw_l[:, 0] * shift[0] + uvw_l[:, 1] * shift[1]))
+    model = rng.standard_normal((2, 3, h, w)).astype(np.float32)
+    want, want_v = [], []
+    for k in range(3):
+        o = oracle.RefGridder(w, h, dl, dl, 1, 7, 63, "float")
+        o.set_is_complex(k == 2)
+        o.set_denormal_phase_centre(*shift)
+        o.prepare_w_layers(nw, 1e12, 0.0, maxw)
+        o.start_inversion_pass(0)
+        o.add_samples(uvw_l, (vis[:, :, k].reshape(-1) * ph).astype(np.complex64))
+        o.finish_inversion_pass()
+        o.finalize_image(1.0)
+        want += list(o.image(imag=True)) if k == 2 else [o.image()]
+        o = oracle.RefGridder(w, h, dl, dl, 1, 7, 63, "float")
+        o.set_is_complex(k == 2)
+        o.set_denormal_phase_centre(*shift)
+        o.prepare_w_layers(nw, 1e12, 0.0, maxw)
+        o.initialize_prediction(model[0, k], model[1, k] if k == 2 else None)
+        o.start_prediction_pass(0)
+        want_v.append(o.sample(uvw_l) * np.conj(ph))
+    kw = dict(precision=precision, n_images=3, complex_images=(2,), l_shift=shift[0],
+              m_shift=shift[1], rotate_visibilities=True, work_chunk=37)
+
+    def compare(re, im):
+        for got, img in zip((re[0], re[1], re[2], im[2]), want):
+            assert rel(got, img) < TOL[precision]
+
+    g = wsclean_amd.WStackingGridder(w, h, dl, dl, 7, 63, **kw)
+    g.prepare_w_layers(nw, 0.0, 0.0, maxw)
+    g.start_inversion_pass(0)
+    g.add_data(uvw[:300], wl, vis[:300])
+    g.add_data(uvw[300:], wl, vis[300:])
+    g.finish_inversion_pass()
+    compare(*g.finalize_image(1.0))
+    g.close()
+    d_uvw, d_wl = torch.from_numpy(uvw).to(dev), torch.from_numpy(wl).to(dev)
+    d_vis, d_model = torch.from_numpy(vis).to(dev), torch.from_numpy(model).to(dev)
+    for passes, max_mem in ((1, 0.0), (2, w * h * 8.0 * 3 * 3)):
+        g = wsclean_amd.DeviceGridder(w, h, dl, dl, 7, 63, **kw)
+        assert g.prepare_w_layers(nw, 0.0, maxw, max_mem=max_mem) == passes
+        g.plan(d_uvw, d_wl)
+        re = torch.zeros((3, h, w), dtype=torch.float32, device=dev)
+        im = torch.zeros_like(re)
+        g.invert(d_vis, 1.0, re, im)
+        out = torch.empty_like(d_vis)
+        g.predict(d_model[0], d_model[1], out)
+        stats = g.stats()
+        assert stats["tiles_total"] == nw * 8 * 4 and stats["chunks"] > stats["bins_used"]
+        compare(re.cpu().numpy(), im.cpu().numpy())
+        for k in range(3):
+            got, ok = out[:, :, k].cpu().numpy().reshape(-1), np.isfinite(want_v[k])
+            assert np.array_equal(ok, np.isfinite(got)) and ok.any()
+            assert rel(got[ok], want_v[k][ok]) < TOL[precision]
+        g.close()
+
+
+@pytest.mark.parametrize("oversampling,tiles", [(63, 16), (221, 16), (223, 9), (1023, 9)])
+def test_cut_tiles_need_the_padded_table_in_lds(oversampling, tiles):
+    """Tiles of 20 keep dividing 60 x 60 where the zero-padded kernel table does
+    not fit the LDS (the oversampling is odd; 221 is the last that fits)."""
+    import wsclean_amd
+    dev = torch.device("cuda:0")
+    g = wsclean_amd.DeviceGridder(60, 60, 0.004, 0.004, 7, oversampling)
+    g.prepare_w_layers(2, 0.0, 1.0)
+    g.plan(torch.zeros((4, 3), dtype=torch.float64, device=dev),
+           torch.ones(1, dtype=torch.float64, device=dev))
+    assert g.stats()["tiles_total"] == 2 * tiles
+    g.close()
