@@ -32,6 +32,11 @@ def test_degridding_launches_whole_rounds_of_resident_workgroups(rule):
         assert per % max(r, 1) == 0 and per >= 5 and per - max(r, 1) < 5
 
 
-def test_runtime_radix_transforms_run_fused_at_long_lines_only(rule):
+def test_runtime_radix_transforms_run_fused_where_they_fill_the_chip(rule):
     sizes = [60, 300, 600, 840, 1260, 1500, 1600, 1680, 1920, 3072, 6144]
-    assert rule([f"fusedRuntimeRadix({n})" for n in sizes]) == [int(n >= 1600) for n in sizes]
+    want = [int(n >= 1600) for n in sizes]
+    assert rule([f"fusedModelRows({n}, 300)" for n in sizes]) == [int(n >= 1400) for n in sizes]
+    assert rule(["fusedModelRows(300, 1800)", "fusedModelRows(480, 3000)"]) == [0, 1]
+    assert rule([f"fusedColumns({n}, 1)" for n in sizes]) == want
+    assert rule(["fusedColumns(480, 3)", "fusedColumns(960, 3)", "fusedColumns(512, 6)",
+                 "fusedColumns(1200, 2)"]) == [0, 1, 1, 0]

@@ -185,7 +185,7 @@ hws_status fft2dGeneric(hws_gridder* g, float2* data, int nbatch, int sign,
   } else {
     // (the mixed precision: the reference precision's terms leave no registers
     // for the cells it keeps)
-    if (model && sparse && sparse->colNeed && fusedRuntimeRadix(W) &&
+    if (model && sparse && sparse->colNeed && fusedModelRows(W, H) &&
         model->precision != HWS_PRECISION_REFERENCE)
       launchModelLayersGeneric(tr, rl, dim3(H >> rbShift), ldsR, st, data, W, H, nbatch, radR,
                                twRow, msrc, sparse->colNeed, sparse->tshift);

@@ -265,7 +265,11 @@ size_t colsProjectGenericLds(int H, int nLayersInPass, int tilesY) {
 
 bool colsProjectGenericSupported(const hws_gridder* g, int nLayersInPass, size_t maxLds) {
   const int t = threadsFor(g->colPlan, 1, true);
-  return fusedRuntimeRadix(g->H) && t != 0 && t <= 512 &&
+  // (the kinds are launched one after the other: the smaller counts)
+  int images = kMaxImages;
+  for (const KindPlan& kp : g->plan.kinds)
+    if (kp.active) images = std::min(images, kp.nImg);
+  return fusedColumns(long(g->W) * images, (t + 63) / 64) && t != 0 && t <= 512 &&
          colsProjectGenericLds(g->H, nLayersInPass, g->plan.tilesY) <= maxLds;
 }
 
