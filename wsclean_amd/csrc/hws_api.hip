@@ -429,10 +429,10 @@ hws_status hws_create(const hws_config* c, hws_gridder** out) {
   if ((st = makeFftPlan(g, g->H, g->colPlan)) != HWS_OK) return bail(st);
   if (g->blocked && !(fastBlockedSize(g->W) && fastBlockedSize(g->H)) && !blockedGenericFits(g))
     g->blocked = false;
-  // uv tile edge of the binned forms: divides W and H, a multiple of 4, at
-  // least K - 1 (a footprint then spans at most two tiles per axis) and with
-  // T + K - 1 <= 64 (6-bit record offsets); 16 (the matrix-core grid
-  // kernel's tile) unless the caller names one
+  // uv tile edge of the binned forms: divides W and H (or is 16, the last tile
+  // cut, see below), a multiple of 4, at least K - 1 (a footprint then spans at
+  // most two tiles per axis) and with T + K - 1 <= 64 (6-bit record offsets); 16
+  // (the matrix-core grid kernel's tile) unless the caller names one
   {
     const int K = g->K;
     const int want = c->tile_size ? int(c->tile_size) : 16;

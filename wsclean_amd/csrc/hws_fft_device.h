@@ -192,7 +192,7 @@ __device__ __forceinline__ size_t blockedAddr(int pos, int f, int W) {
 // not read, and need not have been written); otherwise they are not written.
 // The layer cell (x, y) of a forward transform computed from the model image
 // (the arithmetic of imageToLayersKernel, so the results are identical). REF:
-// the reference precision (float n', FP64 sincos).
+// the reference precision (float n', FP64 sine and cosine).
 template <bool REF>
 __device__ __forceinline__ float2 modelCell(const ModelSource& ms, double w, int x, int y, int W,
                                            int H) {
@@ -212,7 +212,7 @@ __device__ __forceinline__ float2 modelCell(const ModelSource& ms, double w, int
 
 // Layers per workgroup of the model-fed rows pass: the workgroup reads the
 // model rows of its row block once from memory and then from the L2 (the
-// reference precision's FP64 sincos leaves no registers for that: one).
+// reference precision one: four take 128 registers for its 80).
 template <bool REF>
 constexpr int modelLayers() {
   return REF ? 1 : 4;

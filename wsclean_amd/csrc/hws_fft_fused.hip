@@ -14,8 +14,10 @@ namespace {
 // the layer-independent twiddles, and the one wave left per SIMD waits out
 // every LDS access and barrier: at 2048^2 with 32 layers the fused columns of
 // two real images took 1108 us and take 682, the model rows 547 and 486 us an
-// image (reference precision: 1410 -> 818 and 690 -> 550). Three waves (168
-// registers) spill the sums.
+// image (reference precision: 1410 -> 818 and 690 -> 550). The twiddles that no
+// longer fit spill: 14 to 58 values of the fused columns from 512 up (20 at 2048
+// for real images in the mixed precision, 56 for complex ones). Three waves (168
+// registers) spill the sums too.
 #define HWS_TWO_WAVES __attribute__((amdgpu_waves_per_eu(2, 2)))
 
 // Backward columns pass (after fftRowsBlockedSparseKernel) fused with
@@ -333,7 +335,7 @@ bool launchModelLayersPow2(hws_gridder* g, float2* data, int nbatch, const float
   const int W = g->W, H = g->H;
   const bool ref = model.precision == HWS_PRECISION_REFERENCE;
   const bool cplx = model.cplx != 0;
-  // Small images do not fill the chip with one workgroup per row pair
+  // Small images do not fill the chip with one workgroup per row block
   // (1024^2: one wave per SIMD), so the layers are dealt to as many groups of
   // workgroups as bring kModelWaves waves, in groups of at least two layers (a
   // group computes its rows' n' anew, about the time of one layer).

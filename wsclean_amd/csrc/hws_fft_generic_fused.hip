@@ -106,13 +106,15 @@ fftRowsModelLayersGenericKernel(float2* __restrict__ data, int W, int H, int nba
 // added (Kahan) to its pixel's sums, which stay in registers with the
 // pixel's n' (the cells of the last stage's slots). Cells of tile rows
 // without samples read as zero. Every term is computed and added as
-// projectKernel computes and adds it. grid (W / 1, images of the kind);
+// projectKernel computes and adds it. grid (W, images of the kind);
 // dynamic LDS: the transform buffer, then the row bits of the pass's layers.
-// Real images keep to 128 registers (a few spills outside the layer loop) and
-// take the closest multiple of 64 threads, so that two workgroups share a CU at
-// the large sizes: with 142 registers and a power of two of threads one did, and
-// 6144^2 x 96 layers took 28.1 ms against 21.8. Complex images hold twice the
-// sums (206 registers; 128 would spill them).
+// Real images keep to 128 registers (82 values spill in the mixed precision, 78 in
+// the reference one: 52 and 60 bytes of scratch a lane) and take the closest
+// multiple of 64 threads, so that two workgroups share a CU at the large sizes:
+// with 142 registers and a power of two of threads one did, and 6144^2 x 96 layers
+// took 28.1 ms against 21.8; in the reference precision the invert of one image at
+// 3072^2 x 48 layers took 3.96 ms and takes 2.23. Complex images hold twice the sums
+// (206 registers; 128 would spill them).
 template <bool REF, bool CPLX>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(CPLX ? 2 : 4)))
 fftColsProjectGenericKernel(ColsProjectArgs a, const float2* __restrict__ layers,

@@ -482,7 +482,7 @@ struct hws_gridder {
   hipEvent_t ev[8] = {};
   hws_stats stats{};
   int lastOp = 0;  // 1 invert, 2 predict (device one-call forms)
-  int tileSize = 32;  // uv tile edge of the binned forms (divides W and H)
+  int tileSize = 32;  // uv tile edge of the binned forms (16: the last tile may be cut)
 };
 
 namespace hws {

@@ -211,7 +211,8 @@ struct KindArgs {
 // The uv tiles a sample's footprint touches. Footprint cells run from
 // (xs, ys) (centre minus K/2, wrapped into the grid) for K cells per axis;
 // with tileSize >= K - 1 and tiles dividing the grid (or the last one at least
-// K - 1 wide) they touch at most two tiles per axis: tile A holding the first cell and, if different, tile B
+// K - 1 wide) they touch at most two tiles per axis: tile A holding the first
+// cell and, if different, tile B
 // holding the last (possibly wrapped round to tile 0). For each tile the
 // footprint start relative to the tile origin is xo in [-(K-1), T).
 struct TileSpan {
@@ -872,7 +873,7 @@ __device__ __forceinline__ float2 weighted(const GridArgs& a, float2 v, uint32_t
 // (gridding/msgridderbase.cpp:692-704) with shiftFactor = sign * 2 pi
 // (u l_shift + v m_shift) and rad = shiftFactor / lambda. The argument is
 // FP64; the mixed precision reduces it to a fraction of a turn in FP64 and
-// takes the FP32 turnSinCos, the reference precision an FP64 sincos.
+// takes the FP32 turnSinCos, the reference precision turnSinCos64.
 __device__ __forceinline__ float2 rotationPhasor(const GridArgs& a,
                                                  const double* __restrict__ uvw,
                                                  const double* __restrict__ wl, uint32_t idx,
@@ -1222,7 +1223,7 @@ __host__ __device__ inline bool cellTablePadded(int K, int OS, int T) {
 // yKernel[dy] * xKernel[dx] (gridding/wstackinggridder.cpp:560-597). With
 // the zero-padded table (PAD) a cell outside the footprint reads a zero, so
 // the loop has no tests at all. ROT applies the phase-centre rotation (a
-// separate instance: its FP64 sincos costs registers). The sums stay in
+// separate instance: its phasors cost registers). The sums stay in
 // registers for the whole
 // item: no LDS traffic but the kernel table, no read-modify-write chains, no
 // atomics. Item 0 of a bin writes the tile to the layer (ACCUM adds to it);
@@ -2213,7 +2214,7 @@ __device__ __forceinline__ void degridItemRecords(const GridArgs& a, const WorkI
   if (lane < qn) degridRecord<NIMG, KK>(a, queue[lane], kt, sub, a.sg, byOS, out);
 }
 
-// Degridding of one image kind, one work item per workgroup at a time: the
+// Degridding of images of one kind, one work item per workgroup at a time: the
 // (T + K - 1)^2 subgrid around the item's (layer, tile) is gathered from the
 // layer into LDS. Only the primary record of a footprint (the record of the
 // tile holding the footprint start) is degridded, so each wave first
@@ -2984,8 +2985,11 @@ hws_status buildPlan(hws_gridder* g, size_t nrow, size_t nchan,
                        pl.rowKeys, pl.rowOrder);
     HWS_TRY(checkHip(g, hipGetLastError(), "row key launch"));
     // (a few thousand rows are binned as they come: their sort takes six to
-    // twelve launches, about 60 us, and saves less in the binning's atomics:
-    // 2016 rows x 16 channels, the scatter takes 12 us either way)
+    // twelve launches, about 60 us, and saves less in the binning's atomics
+    // however many channels a row has. Plan sorted and not, 2016 rows of 1, 16
+    // and 256 channels: 185, 184, 211 and 146, 137, 164 us; 4032 rows of 16, 256, 1000
+    // and 4000: 196, 231, 321, 627 and 148, 172, 256, 565; invert and predict take
+    // the same with either order)
     if (nrow > kUnsortedRows) {
       int keyBits = 1;  // keys run from 0 to nbins
       while (keyBits < 32 && (size_t(1) << keyBits) <= pl.nbins) ++keyBits;
