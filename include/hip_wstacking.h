@@ -97,10 +97,11 @@ typedef struct hws_config {
    * does (gridding/wsmsgridder.cpp:185-190, 328-332). 0: only the n' shift
    * of WStackingGridder::SetDenormalPhaseCentre. */
   int rotate_visibilities;
-  /* uv tile edge for binning; 0 = 16 where it divides the image or (oversampling up
-   * to 221 at kernel size 7) leaves a last tile of kernel_size - 1 cells, else the edge closest to 16
-   * that divides it (16: the matrix-core grid kernel; 8: the VALU cell kernel;
-   * other edges: the private-tile kernel over origin-sorted records). */
+  /* uv tile edge for binning; 0 = 16 where it divides the image or (oversampling
+   * up to 221 at kernel size 7) leaves a last tile of kernel_size - 1 cells or
+   * more, else the edge closest to 16 that divides it (16: the matrix-core grid
+   * kernels; 8: the VALU cell kernel; other edges: the private-tile kernel over
+   * origin-sorted records). */
   size_t tile_size;
   /* Records per work item of the binned grid/degrid kernels: a (layer, tile)
    * bin with more records is split into several items (whose tiles are
