@@ -143,7 +143,7 @@ def test_sums_of_dense_bins_keep_their_precision(oracle, w, precision):
 @pytest.mark.parametrize("w,h", [(120, 60), (64, 96)])
 def test_degridding_of_one_to_four_images(oracle, w, h, K):
     """The kernel sizes and image counts of the degridding kernel, footprints
-    about every tile edge (60 and 120 leave a cut tile up to K = 9 and K = 13)."""
+    about every tile edge (120 x 60 has cut tiles up to K = 9)."""
     import wsclean_amd
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(w + K)
